@@ -6,7 +6,7 @@
 // through nvsubquadratic/modules/subq_ops_causal_conv1d.py:77-83.
 #include <mutex>
 
-#include "direct_conv.h"
+#include "toeplitz_mma.h"
 
 namespace nsq {
 
@@ -18,7 +18,7 @@ namespace nsq {
 constexpr size_t kNoAllocScratchBytes = NSQ_NOALLOC_SCRATCH_BYTES;
 static __device__ __align__(256) float scratch[kNoAllocScratchBytes / sizeof(float)];
 
-// Forward for K <= 16 taps from registers: thread t of a tile owns outputs
+// Forward for up to 16 taps (short_fwd) from registers: thread t of a tile owns outputs
 // n = n0 + 8t + e, e < 8; with the taps left-padded to KP = 4, 8 or 16,
 // y[n] = act(bias + sum_j wk[j] x[n - KP + 1 + j]).  Its x window
 // [n0 + 8t - 8 XB, n0 + 8t + 8) comes straight from HBM in aligned chunks of 8
@@ -59,172 +59,33 @@ __global__ __launch_bounds__(kConvThreads) void cconv_fwd_short_kernel(const typ
   store8<DT, AL>(RowBuf<DT, AL>(y + row * L, L), base, out);
 }
 
-// ---------------------------------------------------------------------------
-// Matrix-core path (K >= 16; used above 16 taps): a workgroup walks a segment of
-// kConvSegTiles tiles of one (b, c) row; per tile the source window (fp32,
-// in the split layout ToeplitzMfma reads) is staged from registers loaded during the
-// previous tile, the MFMA band gives acc[p] for the tile's 2048 outputs, and
-// the epilogue stores from the accumulator layout through a range-checked row
-// buffer.  Modes:
-//   FWD (ACT identity / silu): src = x from n0 - K + 1, y = act(acc + bias);
-//   GPRE: the same conv, out (fp32) = gy * silu'(acc + bias);
-//   CORR: src = gp from n0 on the reversed band, gx = acc
-//         (gx[n] = sum_j w[j] gp[n + K - 1 - j]).
-// ---------------------------------------------------------------------------
-enum { CC_FWD_ID = 0, CC_FWD_SILU = 1, CC_GPRE = 2, CC_CORR = 3 };
-constexpr int kConvSegTiles = 4;
-
-template <int DS, int DO, int NS, int MODE>
-__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(3))) void cconv_mfma_kernel(
-    const typename Elem<DS>::T* __restrict__ src, const float* __restrict__ w, const float* __restrict__ bias,
-    const typename Elem<DO>::T* __restrict__ gy, void* __restrict__ out, int C, int L, int K) {
-  constexpr int ZW = mfma_src_count<NS>();
-  constexpr int ZR = win_half(ZW);
-  __shared__ __align__(16) float zp[win_words(ZW)];
-  __shared__ __align__(16) float wl[kConvWeightFloats];
-  const int64_t row = blockIdx.x;
-  const int c = int(row % C);
-  const int ntiles = (L + kConvTile - 1) / kConvTile;
-  const int t_begin = int(blockIdx.y) * kConvSegTiles;
-  const int t_end = min(ntiles, t_begin + kConvSegTiles);
-  const int t = int(threadIdx.x);
-  constexpr bool CORR = MODE == CC_CORR;
-  if (CORR)
-    stage_weights<true>(wl, w + int64_t(c) * K, K);
-  else
-    stage_weights<false>(wl, w + int64_t(c) * K, K);
-  const int shift = CORR ? 0 : K - 1;  // window word m is src[n0 - shift + m]
-  RowStage<DS, ZW> sw;
-  sw.load(src + row * L, int64_t(t_begin) * kConvTile - shift, 0, L);
-  __syncthreads();  // weights staged
-  ToeplitzMfma<NS> tm;
-  tm.load_weights(wl, K);
-  const float b0 = (!CORR && bias) ? bias[c] : 0.f;
-  const RowBuf<DO, false> ob((typename Elem<DO>::T*)out + row * L, L);
-  const RowBuf<NSQ_DTYPE_F32, false> ofb((float*)out + row * L, L);
-  const RowBuf<DO, false> gyb(gy + row * L, L);
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63;
-  for (int ti = t_begin; ti < t_end; ++ti) {
-    const int64_t n0 = int64_t(ti) * kConvTile;
-#pragma unroll
-    for (int it = 0; it < RowStage<DS, ZW>::IT; ++it) {
-      const int m = t + it * kConvThreads;
-      if (m < ZW) zp[win_at(m, ZR)] = RowBuf<DS, false>::bits_to_f32(sw.v[it]);
-    }
-    __syncthreads();
-    if (ti + 1 < t_end) sw.load(src + row * L, n0 + kConvTile - shift, 0, L);
-    nsq_f32x4_t acc0, acc1;
-    tm.run2(zp, ZR, 16 * wave, 16 * (wave + kConvWaves), acc0, acc1);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int p = 16 * (16 * (wave + h * kConvWaves) + 4 * (l >> 4) + r) + (l & 15);
-        const float a = (h ? acc1[r] : acc0[r]) + b0;
-        if constexpr (MODE == CC_FWD_ID) {
-          ob.store_elem(n0 + p, a);
-        } else if constexpr (MODE == CC_FWD_SILU) {
-          ob.store_elem(n0 + p, act_fwd<NSQ_ACT_SILU>(a));
-        } else if constexpr (MODE == CC_GPRE) {
-          ofb.store_elem(n0 + p, gyb.elem(n0 + p) * dsilu(a));
-        } else {
-          ob.store_elem(n0 + p, a);
-        }
-      }
-    }
-    __syncthreads();
-  }
+// Whole rows of 16-byte chunks: every row starts 16-byte aligned and ends on a chunk.
+template <int DT>
+static bool rows16(int64_t L, const void* a, const void* b, const void* c) {
+  return L % (DT == NSQ_DTYPE_F32 ? 4 : 8) == 0 &&
+         ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 15) == 0;
 }
 
-// Weight / bias gradients on the matrix cores (K >= 16; used above 16 taps): per tile,
-//   D[i][t] += sum_a gp[16a + i] * xwin[16a + t],  xwin[m] = x[n0 - K + 1 + m],
-// gw[j] = sum_i D[i][i + j] over the workgroup's tiles (one channel, a segment
-// of its (b, tile) sequence), gb = sum gp; fixed-order reduction into a
-// per-workgroup partial [K + 1], summed by cconv_wgrad_reduce_kernel.
-template <int DG, int DX, int NS>
-__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2))) void cconv_wgrad_mfma_kernel(
-    const typename Elem<DG>::T* __restrict__ gp, const typename Elem<DX>::T* __restrict__ x, float* __restrict__ part,
-    int B, int C, int L, int K) {
-  constexpr int ZW = mfma_src_count<NS>();
-  constexpr int ZR = win_half(ZW);
-  constexpr int ZWORDS = win_words(ZW);
-  constexpr int TG = NS / 4;
-  constexpr int RW = 4 * NS;
-  static_assert(16 * RW <= ZWORDS + kConvTile, "cconv_wgrad_mfma_kernel: reduction area");
-  __shared__ __align__(16) float sm[ZWORDS + kConvTile];
-  float* zp = sm;
-  float* gs = sm + ZWORDS;  // gp of the tile, plain
-  const int c = int(blockIdx.x);
-  const int ntiles = (L + kConvTile - 1) / kConvTile;
-  const int g_begin = int(blockIdx.y) * kConvSegTiles;
-  const int g_end = min(B * ntiles, g_begin + kConvSegTiles);
-  const int t = int(threadIdx.x);
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63;
-  const int kk = l >> 4, li = l & 15;
-  nsq_f32x4_t D[TG];
-#pragma unroll
-  for (int tg = 0; tg < TG; ++tg) D[tg] = nsq_f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float bacc = 0.f;
-  for (int g = g_begin; g < g_end; ++g) {
-    const int b = g / ntiles, ti = g - b * ntiles;
-    const int64_t row = int64_t(b) * C + c;
-    const int64_t n0 = int64_t(ti) * kConvTile;
-    {
-      RowStage<DX, ZW> sx;
-      RowStage<DG, kConvTile> sg;
-      sx.load(x + row * L, n0 - (K - 1), 0, L);
-      sg.load(gp + row * L, n0, 0, L);
-#pragma unroll
-      for (int it = 0; it < RowStage<DX, ZW>::IT; ++it) {
-        const int m = t + it * kConvThreads;
-        if (m < ZW) zp[win_at(m, ZR)] = RowBuf<DX, false>::bits_to_f32(sx.v[it]);
-      }
-      sg.store(gs, kConvTile);
-#pragma unroll
-      for (int it = 0; it < RowStage<DG, kConvTile>::IT; ++it) bacc += RowBuf<DG, false>::bits_to_f32(sg.v[it]);
-    }
-    __syncthreads();
-    // win_at(16 (a0 + kk + tg) + li) = win_at(16 kk + li) + 8 (a0 + tg)
-    const float* zl = zp + win_at(16 * kk + li, ZR);
-#pragma unroll 2
-    for (int a0 = 32 * wave; a0 < 32 * wave + 32; a0 += 4) {
-      const float av = gs[16 * (a0 + kk) + li];
-#pragma unroll
-      for (int tg = 0; tg < TG; ++tg) {
-        const float bv = zl[8 * (a0 + tg)];
-        D[tg] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, D[tg], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-  }
-  float* red = sm;
-  for (int w = 0; w < kConvWaves; ++w) {
-    if (wave == w) {
-#pragma unroll
-      for (int tg = 0; tg < TG; ++tg)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float& dst = red[(4 * kk + r) * RW + 16 * tg + li];
-          dst = (w == 0 ? 0.f : dst) + D[tg][r];
-        }
-    }
-    __syncthreads();
-  }
-  const int nparts = int(gridDim.y);
-  float* pw = part + (int64_t(c) * nparts + blockIdx.y) * (K + 1);
-  if (t < K) {
-    float sacc = 0.f;
-    for (int i = 0; i < 16; ++i) sacc += red[i * RW + i + t];
-    pw[t] = sacc;
-  }
-  __syncthreads();
-  red[t] = bacc;  // bias partial: fixed-order sum over the threads
-  __syncthreads();
-  if (t == 0) {
-    float sacc = 0.f;
-    for (int i = 0; i < kConvThreads; ++i) sacc += red[i];
-    pw[K] = sacc;
-  }
+constexpr int kConvSegTiles = 4;  // tiles per workgroup of the register backward
+// The register kernels run up to 4 taps, the matrix-core ones above 16; between, by what measured faster (us, register /
+// matrix-core).  B=4 C=4096 L=8192 (2^27 samples):
+//   forward, bf16:  identity K = 8 93 / 101, K = 9 112 / 101;  silu K = 4 117 / 105, K = 5 135 / 105;
+//   forward, fp32:  K = 4 198 / 201, K = 5 218 / 201, K = 16 226 / 201 (either activation);
+//   backward, bf16: silu K = 4 196 / 218, K = 5 274 / 218;  fp32: silu K = 4 339 / 317, K = 5 417 / 317.
+// Below 2^25 samples with aligned rows the matrix-core kernels' setup (bands, staging) shows, in fp32 up to 16 taps
+// forward (B=4 C=1024 L=2048, silu: K = 16 13.2 / 14.3) and 8 backward (K = 7 25.6 / 27.2), in 16 bits up to 8 forward
+// (K = 7 9.4 / 11.1); unaligned rows favour them from 5 taps (B=8 C=768 L=777 fp32, K = 7 25.8 / 18.0).
+constexpr int kConvShortMax = 4;
+constexpr int64_t kConvSmall = int64_t(1) << 25;
+template <int DT>
+static bool short_fwd(int K, int act, int64_t samples, bool aligned) {
+  constexpr bool F32 = DT == NSQ_DTYPE_F32;
+  return K <= kConvShortMax || (K <= 8 && act == NSQ_ACT_IDENTITY && !F32) ||
+         (K <= (F32 ? 16 : 8) && aligned && samples < kConvSmall);
+}
+template <int DT>
+static bool short_bwd(int K, int64_t samples, bool aligned) {
+  return K <= kConvShortMax || (DT == NSQ_DTYPE_F32 && K <= 8 && aligned && samples < kConvSmall);
 }
 
 __global__ void cconv_wgrad_reduce_kernel(const float* __restrict__ part, int nparts, int K, float* __restrict__ gw,
@@ -244,52 +105,403 @@ static int64_t cconv_wgrad_parts(int64_t B, int64_t L) {
   return ceil_div(B * ceil_div(L, kConvTile), kConvSegTiles);
 }
 
-template <int DT, int NS>
-static void launch_fwd_mfma(const void* x, const float* w, const float* bias, void* y, int act, int B, int C, int L,
-                            int K, hipStream_t st) {
-  using ET = typename Elem<DT>::T;
-  dim3 grid(B * C, unsigned(ceil_div(ceil_div(L, kConvTile), kConvSegTiles)));
-  if (act == NSQ_ACT_SILU)
-    hipLaunchKernelGGL((cconv_mfma_kernel<DT, DT, NS, CC_FWD_SILU>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
-                       bias, (const ET*)nullptr, y, C, L, K);
-  else
-    hipLaunchKernelGGL((cconv_mfma_kernel<DT, DT, NS, CC_FWD_ID>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
-                       bias, (const ET*)nullptr, y, C, L, K);
+// ---------------------------------------------------------------------------
+// Matrix-core path (more than kConvShortMax taps): banded Toeplitz products
+// at fp32 precision on the bf16 matrix cores (toeplitz_mma.h).  A workgroup
+// owns one channel and walks a run of its (batch row, 2048-output tile)
+// sequence, so the split taps are prepared once per run.
+// ---------------------------------------------------------------------------
+constexpr int kMmaTarget = 4096;  // workgroups wanted: 4 or more per resident slot (256 CUs x 2..4)
+
+// Tiles per run: as many as leave kMmaTarget workgroups, at least 1.
+static int64_t mma_run_tiles(int64_t B, int64_t C, int64_t L) {
+  const int64_t tiles = B * ceil_div(L, kConvTile), want = ceil_div(kMmaTarget, C);
+  return tiles / want > 1 ? tiles / want : 1;
+}
+static int64_t mma_runs(int64_t B, int64_t C, int64_t L) {
+  return ceil_div(B * ceil_div(L, kConvTile), mma_run_tiles(B, C, L));
 }
 
-template <int DT, int NS>
-static void launch_bwd_mfma(const void* gy, const void* x, const float* w, const float* bias, void* gx, float* gw,
-                            float* gb, int act, int B, int C, int L, int K, float* ws, hipStream_t st) {
-  using ET = typename Elem<DT>::T;
-  dim3 grid(B * C, unsigned(ceil_div(ceil_div(L, kConvTile), kConvSegTiles)));
-  const int64_t nparts = cconv_wgrad_parts(B, L);
-  dim3 wgrid(C, unsigned(nparts));
-  if (act == NSQ_ACT_SILU) {
-    float* gpre = ws;
-    float* part = ws + int64_t(B) * C * L;
-    hipLaunchKernelGGL((cconv_mfma_kernel<DT, DT, NS, CC_GPRE>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
-                       bias, (const ET*)gy, (void*)gpre, C, L, K);
-    hipLaunchKernelGGL((cconv_mfma_kernel<NSQ_DTYPE_F32, DT, NS, CC_CORR>), grid, dim3(kConvThreads), 0, st,
-                       (const float*)gpre, w, (const float*)nullptr, (const ET*)nullptr, gx, C, L, K);
-    hipLaunchKernelGGL((cconv_wgrad_mfma_kernel<NSQ_DTYPE_F32, DT, NS>), wgrid, dim3(kConvThreads), 0, st,
-                       (const float*)gpre, (const ET*)x, part, B, C, L, K);
-    hipLaunchKernelGGL(cconv_wgrad_reduce_kernel, dim3(C), dim3(kConvThreads + 64), 0, st, (const float*)part,
-                       int(nparts), K, gw, gb);
-  } else {
-    float* part = ws;
-    hipLaunchKernelGGL((cconv_mfma_kernel<DT, DT, NS, CC_CORR>), grid, dim3(kConvThreads), 0, st, (const ET*)gy, w,
-                       (const float*)nullptr, (const ET*)nullptr, gx, C, L, K);
-    hipLaunchKernelGGL((cconv_wgrad_mfma_kernel<DT, DT, NS>), wgrid, dim3(kConvThreads), 0, st, (const ET*)gy,
-                       (const ET*)x, part, B, C, L, K);
-    hipLaunchKernelGGL(cconv_wgrad_reduce_kernel, dim3(C), dim3(kConvThreads + 64), 0, st, (const float*)part,
-                       int(nparts), K, gw, gb);
+// The products of S steps for the 16-block M-tiles at blocks a0 and a1: src holds P part arrays of `stride` elements.
+template <int S, int P>
+__device__ __forceinline__ void band_run2(const nsq_bf16x8_t (&tap)[S][kTapParts], const uint16_t* src, int stride,
+                                          int a0, int a1, nsq_f32x4_t& c0, nsq_f32x4_t& c1) {
+  const int l = int(threadIdx.x) & 63, kk = l >> 4, a = l & 15;
+  const uint16_t* p0 = src + 16 * (a0 + a) + 8 * kk;
+  const uint16_t* p1 = src + 16 * (a1 + a) + 8 * kk;
+  c0 = nsq_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  c1 = nsq_f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    nsq_bf16x8_t u[P], v[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int o = p * stride + 32 * s;
+      if (band_half_last<S>() && s == S - 1) {  // the window ends 16 columns before the step does
+        const bool z = kk >= 2;
+        const uint4 zero = make_uint4(0, 0, 0, 0);
+        u[p] = as_bf16x8(z ? zero : *reinterpret_cast<const uint4*>(p0 + (z ? 0 : o)));
+        v[p] = as_bf16x8(z ? zero : *reinterpret_cast<const uint4*>(p1 + (z ? 0 : o)));
+      } else {
+        u[p] = as_bf16x8(*reinterpret_cast<const uint4*>(p0 + o));
+        v[p] = as_bf16x8(*reinterpret_cast<const uint4*>(p1 + o));
+      }
+    }
+    mma_parts<P>(tap[s], u, c0);
+    mma_parts<P>(tap[s], v, c1);
   }
 }
 
+// y = act(conv + bias).  Bound by HBM (x in, y out) from K = 128 down: 15 MFMAs of 16 cycles per 256 outputs are
+// 60 us at B=4 C=4096 L=8192 bf16, where x and y take 100 us at 5.3 TB/s.  Measured there: 101 us at K = 17, 120 at
+// K = 128 (152 with silu), 183 at K = 256; the fp32 matrix products before took 409 us at K = 128 with silu.  The window of a tile (KP + 2048 samples as bf16
+// parts) is double-buffered in LDS, one barrier per tile, the next tile's samples in flight during the products.
+template <int DT, int S, int ACT, bool AL>
+__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(S <= 5 ? 4 : 2))) void
+cconv_fwd_mma_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __restrict__ w,
+                     const float* __restrict__ bias, typename Elem<DT>::T* __restrict__ y, int B, int C, int L, int K,
+                     int run) {
+  constexpr int KP = band_kp<S>(), W = KP + kConvTile, P = kParts<DT>;
+  // two windows; first the band's operands, made once for the four waves
+  constexpr int BAND = band_operands<S>() * 16, WIN = P * W * 2;
+  __shared__ __align__(16) unsigned char sm[BAND > 2 * WIN ? BAND : 2 * WIN];
+  __shared__ __align__(16) float wl[kConvWeightFloats];
+  uint4* band = reinterpret_cast<uint4*>(sm);
+  const int c = int(blockIdx.x);
+  const int ntiles = (L + kConvTile - 1) / kConvTile;
+  const int g0 = int(blockIdx.y) * run, g1 = min(B * ntiles, g0 + run);
+  const int t = int(threadIdx.x);
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63;
+  stage_weights<false>(wl, w + int64_t(c) * K, K);
+  PartChunk<DT, AL> cm, cx;  // samples [8t, 8t + 8) of the window and, for the first threads, [2048 + 8t, ...)
+  auto load = [&](int g) {
+    const int b = g / ntiles, n0 = (g - b * ntiles) * kConvTile;
+    const RowBuf<DT, false> rb(x + (int64_t(b) * C + c) * L, L);
+    cm.load(rb, n0 - KP + 8 * t);
+    if (t < KP / 8) cx.load(rb, n0 - KP + kConvTile + 8 * t);
+  };
+  load(g0);
+  __syncthreads();  // taps staged
+  put_band<S, false>(band, wl, K);
+  __syncthreads();
+  nsq_bf16x8_t tap[S][kTapParts];
+  get_band<S>(band, tap);
+  __syncthreads();
+  const float b0 = bias ? bias[c] : 0.f;
+  for (int g = g0; g < g1; ++g) {
+    const int b = g / ntiles, n0 = (g - b * ntiles) * kConvTile;
+    uint16_t* xb = reinterpret_cast<uint16_t*>(sm + ((g - g0) & 1) * WIN);
+    uint4 o[P];
+    cm.parts(o);
+#pragma unroll
+    for (int p = 0; p < P; ++p) *reinterpret_cast<uint4*>(xb + p * W + 8 * t) = o[p];
+    if (t < KP / 8) {
+      cx.parts(o);
+#pragma unroll
+      for (int p = 0; p < P; ++p) *reinterpret_cast<uint4*>(xb + p * W + kConvTile + 8 * t) = o[p];
+    }
+    __syncthreads();  // a wave writes this window again two barriers on, when all have read it
+    if (g + 1 < g1) load(g + 1);
+    if (n0 + 512 * wave >= L) continue;
+    nsq_f32x4_t acc[2];
+    band_run2<S, P>(tap, xb, W, 32 * wave, 32 * wave + 16, acc[0], acc[1]);
+    const RowBuf<DT, false> ob(y + (int64_t(b) * C + c) * L, L);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = act_fwd<ACT>(acc[h][r] + b0);
+      store4<DT, AL>(ob, n0 + 16 * (32 * wave + 16 * h + (l & 15)) + 4 * (l >> 4), v);
+    }
+  }
+}
+
+// Whole backward of one channel's run of tiles in one pass (the earlier three kernels wrote gpre as fp32 and read it
+// twice, 20 bytes a sample against 6 here):
+//   gpre = gy silu'(conv(x) + bias) (identity: gy), by the conv band over the tile's 2048 outputs;
+//   gx[n] = sum_j w[j] gpre[n + K - 1 - j], by the reversed band;
+//   D[i][t] += sum_a gpre[16a + i] x[n0 - KP + 16a + t], gw[j] = sum_i D[i][i + j + pad].
+// The tiles of a row run from its end to its start, so the KP positions of gpre past a tile are the first ones of
+// the tile before; a run that starts inside a row computes that tile's gpre once more.
+// LDS: both bands as operands (reloaded into registers per phase: together they would not fit beside D), the window
+// of x and gpre as bf16 parts, in order.  The weight gradient contracts over the blocks a, so its operands are the
+// columns of these arrays' 16-wide rows: the transposing LDS read (tr16_column8) forms them, with no second copy.
+// The weight gradient is fp32 exactly as the bands are (all kept products exact, fp32 sums).
+// Bound by issue: at K = 128 with silu 117 MFMAs and about 400 VALU instructions per wave and tile (gpre, its split)
+// fill 70% of the cycles at 3 waves per SIMD.  B=4 C=4096 L=8192 bf16: 478 us with silu, 201 identity (155 at K = 17:
+// 5.2 TB/s), against 1220 us for the three kernels.
+template <int DT, int S, int ACT>
+struct CconvBwdCfg {
+  static constexpr bool SILU = ACT == NSQ_ACT_SILU;
+  static constexpr int KP = band_kp<S>(), W = KP + kConvTile, TG = KP / 16 + 1;
+  static constexpr int PX = kParts<DT>, PG = SILU ? 3 : PX;
+  static constexpr int TAPS = band_operands<S>();
+  static constexpr int O_REV = 0, O_CONV = O_REV + TAPS * 16, O_XL = O_CONV + (SILU ? TAPS * 16 : 0),
+                       O_GL = O_XL + PX * W * 2, BYTES = O_GL + PG * W * 2;
+  static_assert(16 * 16 * TG * 4 <= TAPS * 16, "cconv_bwd_mma: the final reduction reuses a band");
+};
+
+template <int DT, int S, int ACT, bool AL>
+__global__ __launch_bounds__(kConvThreads)
+__attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 1 : CconvBwdCfg<DT, S, ACT>::BYTES > 53 * 1024 ? 2 : 3))) void cconv_bwd_mma_kernel(
+    const typename Elem<DT>::T* __restrict__ gy, const typename Elem<DT>::T* __restrict__ x,
+    const float* __restrict__ w, const float* __restrict__ bias, typename Elem<DT>::T* __restrict__ gx,
+    float* __restrict__ part, int B, int C, int L, int K, int run) {
+  using F = CconvBwdCfg<DT, S, ACT>;
+  constexpr int KP = F::KP, W = F::W, PX = F::PX, PG = F::PG;
+  constexpr bool SILU = F::SILU;
+  __shared__ __align__(16) unsigned char sm[F::BYTES];
+  uint4* rev = reinterpret_cast<uint4*>(sm + F::O_REV);
+  uint4* conv = reinterpret_cast<uint4*>(sm + F::O_CONV);
+  uint16_t* xl = reinterpret_cast<uint16_t*>(sm + F::O_XL);
+  uint16_t* gl = reinterpret_cast<uint16_t*>(sm + F::O_GL);
+  float* wl = reinterpret_cast<float*>(sm + F::O_GL);  // the taps until the bands are made; at the end wave sums
+  const int c = int(blockIdx.x);
+  const int ntiles = (L + kConvTile - 1) / kConvTile;
+  const int g0 = int(blockIdx.y) * run, g1 = min(B * ntiles, g0 + run);
+  const int t = int(threadIdx.x);
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63;
+  const int kk = l >> 4, li = l & 15;
+  const int pad = KP - K + 1, tg0 = pad >> 4;
+  const float b0 = bias ? bias[c] : 0.f;
+
+  stage_weights<false>(wl, w + int64_t(c) * K, K);
+  PartChunk<DT, AL> xm, xx, gm, gx8;
+  auto row_of = [&](int g) { return (int64_t(g / ntiles) * C + c) * L; };
+  auto load = [&](int g) {
+    const int n0 = (g % ntiles) * kConvTile;
+    const RowBuf<DT, false> rb(x + row_of(g), L);
+    xm.load(rb, n0 - KP + 8 * t);
+    if (t < KP / 8) xx.load(rb, n0 - KP + kConvTile + 8 * t);
+    if constexpr (!SILU) {
+      const RowBuf<DT, false> gb(gy + row_of(g), L);
+      gm.load(gb, n0 + 8 * t);
+      if (t < KP / 8) gx8.load(gb, n0 + kConvTile + 8 * t);
+    }
+  };
+  load(g1 - 1);
+  __syncthreads();  // taps staged
+  put_band<S, true>(rev, wl, K);
+  if constexpr (SILU) put_band<S, false>(conv, wl, K);
+  __syncthreads();
+  auto stage_x = [&]() {
+    uint4 o[PX];
+    xm.parts(o);
+#pragma unroll
+    for (int p = 0; p < PX; ++p) *reinterpret_cast<uint4*>(xl + p * W + 8 * t) = o[p];
+    if (t < KP / 8) {
+      xx.parts(o);
+#pragma unroll
+      for (int p = 0; p < PX; ++p) *reinterpret_cast<uint4*>(xl + p * W + kConvTile + 8 * t) = o[p];
+    }
+  };
+  float bacc = 0.f;
+  // gpre of tile g into gl (SILU)
+  auto make_gpre = [&](int g, bool count) {
+    const int n0 = (g % ntiles) * kConvTile;
+    const RowBuf<DT, false> gb(gy + row_of(g), L);
+    Quad<DT, AL> q[2];
+    const int p0 = 16 * (32 * wave + li) + 4 * kk;  // the lane's positions in M-tile 2 wave; 256 on in the next
+    q[0].load(gb, n0 + p0);
+    q[1].load(gb, n0 + p0 + 256);
+    uint32_t b[2][4][PG];
+    if (n0 + 512 * wave < L) {
+      nsq_bf16x8_t tap[S][kTapParts];
+      get_band<S>(conv, tap);
+      nsq_f32x4_t acc[2];
+      band_run2<S, PX>(tap, xl, W, 32 * wave, 32 * wave + 16, acc[0], acc[1]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float gp = n0 + p0 + 256 * h + r < L ? q[h].at(r) * dsilu(acc[h][r] + b0) : 0.f;
+          if (count) bacc += gp;
+          split_parts<PG>(gp, b[h][r]);
+        }
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int p = 0; p < PG; ++p) b[h][r][p] = 0;
+    }
+#pragma unroll
+    for (int p = 0; p < PG; ++p)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *reinterpret_cast<uint2*>(gl + p * W + p0 + 256 * h) =
+            make_uint2(b[h][0][p] | (b[h][1][p] << 16), b[h][2][p] | (b[h][3][p] << 16));
+  };
+  // gy itself into gl (identity)
+  auto stage_g = [&]() {
+    uint4 o[PX];
+    gm.parts(o);
+#pragma unroll
+    for (int p = 0; p < PX; ++p) *reinterpret_cast<uint4*>(gl + p * W + 8 * t) = o[p];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) bacc += gm.w.at(k);
+    if (t < KP / 8) {
+      gx8.parts(o);
+#pragma unroll
+      for (int p = 0; p < PX; ++p) *reinterpret_cast<uint4*>(gl + p * W + kConvTile + 8 * t) = o[p];
+    }
+  };
+  // the KP positions past the tile: the first KP of the tile after it (or zeros past the row)
+  auto carry = [&](bool zero) {
+    if (t < KP / 8)
+#pragma unroll
+      for (int p = 0; p < PG; ++p)
+        *reinterpret_cast<uint4*>(gl + p * W + kConvTile + 8 * t) =
+            zero ? make_uint4(0, 0, 0, 0) : *reinterpret_cast<const uint4*>(gl + p * W + 8 * t);
+  };
+
+  nsq_f32x4_t D[F::TG];
+#pragma unroll
+  for (int tg = 0; tg < F::TG; ++tg) D[tg] = nsq_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if constexpr (SILU) {
+    if (g1 % ntiles != 0) {  // the run starts inside a row: gpre of the tile after it
+      load(g1);
+      stage_x();
+      __syncthreads();
+      make_gpre(g1, false);
+      load(g1 - 1);
+      __syncthreads();
+    }
+  }
+  for (int g = g1 - 1; g >= g0; --g) {
+    const int n0 = (g % ntiles) * kConvTile;
+    if constexpr (SILU) carry(g % ntiles == ntiles - 1);
+    stage_x();
+    if constexpr (!SILU) stage_g();
+    __syncthreads();
+    if (g > g0) load(g - 1);
+    if constexpr (SILU) {
+      make_gpre(g, true);
+      __syncthreads();
+    }
+    if (n0 + 512 * wave < L) {
+      nsq_bf16x8_t tap[S][kTapParts];
+      get_band<S>(rev, tap);
+      nsq_f32x4_t acc[2];
+      band_run2<S, PG>(tap, gl, W, 32 * wave, 32 * wave + 16, acc[0], acc[1]);
+      const RowBuf<DT, false> ob(gx + row_of(g), L);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float v[4] = {acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
+        store4<DT, AL>(ob, n0 + 16 * (32 * wave + 16 * h + li) + 4 * kk, v);
+      }
+    }
+    {
+      // wave w contracts over blocks 32 w .. 32 w + 31
+      nsq_bf16x8_t ga[PG];
+#pragma unroll
+      for (int p = 0; p < PG; ++p) ga[p] = tr16_column8(gl + p * W + 512 * wave);
+#pragma unroll
+      for (int tg = 0; tg < F::TG; ++tg) {
+        if (tg < tg0) continue;
+        nsq_bf16x8_t xb[PX];
+#pragma unroll
+        for (int p = 0; p < PX; ++p) xb[p] = tr16_column8(xl + p * W + 512 * wave + 16 * tg);
+#pragma unroll
+        for (int d = 2; d >= 0; --d)
+#pragma unroll
+          for (int p = 0; p < PX; ++p)
+            if (d - p >= 0 && d - p < PG)
+              D[tg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[d - p], xb[p], D[tg], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+  // fixed-order sums over the waves, then along the diagonals
+  constexpr int RW = 16 * F::TG;
+  float* red = reinterpret_cast<float*>(sm + F::O_REV);
+  for (int v = 0; v < kConvWaves; ++v) {
+    if (wave == v) {
+#pragma unroll
+      for (int tg = 0; tg < F::TG; ++tg)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float& dst = red[(4 * kk + r) * RW + 16 * tg + li];
+          dst = (v == 0 ? 0.f : dst) + D[tg][r];
+        }
+    }
+    __syncthreads();
+  }
+  float* pw = part + (int64_t(c) * gridDim.y + blockIdx.y) * (K + 1);
+  if (t < K) {
+    float s = 0.f;
+    for (int i = 0; i < 16; ++i) s += red[i * RW + i + pad + t];
+    pw[t] = s;
+  }
+#pragma unroll
+  for (int o = 32; o; o >>= 1) bacc += __shfl_xor(bacc, o);
+  if (l == 0) wl[wave] = bacc;
+  __syncthreads();
+  if (t == 0) pw[K] = (wl[0] + wl[1]) + (wl[2] + wl[3]);
+}
+
+template <class F>
+static void with_band(int64_t K, F&& f) {
+  switch (band_steps_for(K)) {
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    case 5: return f(std::integral_constant<int, 5>{});
+    case 7: return f(std::integral_constant<int, 7>{});
+    default: return f(std::integral_constant<int, 9>{});
+  }
+}
+
+template <int DT>
+static void launch_fwd_mma(const void* x, const float* w, const float* bias, void* y, int act, int B, int C, int L,
+                           int K, hipStream_t st) {
+  using ET = typename Elem<DT>::T;
+  const dim3 grid(C, unsigned(mma_runs(B, C, L)));
+  const int run = int(mma_run_tiles(B, C, L));
+  const bool al = rows16<DT>(L, x, y, nullptr);
+  with_band(K, [&](auto s) {
+    auto go = [&](auto a, auto f) {
+      hipLaunchKernelGGL((cconv_fwd_mma_kernel<DT, decltype(s)::value, decltype(f)::value, decltype(a)::value>), grid,
+                         dim3(kConvThreads), 0, st, (const ET*)x, w, bias, (ET*)y, B, C, L, K, run);
+    };
+    using SILU = std::integral_constant<int, NSQ_ACT_SILU>;
+    using IDN = std::integral_constant<int, NSQ_ACT_IDENTITY>;
+    if (al)
+      act == NSQ_ACT_SILU ? go(std::true_type{}, SILU{}) : go(std::true_type{}, IDN{});
+    else
+      act == NSQ_ACT_SILU ? go(std::false_type{}, SILU{}) : go(std::false_type{}, IDN{});
+  });
+}
+
+template <int DT>
+static void launch_bwd_mma(const void* gy, const void* x, const float* w, const float* bias, void* gx, float* gw,
+                           float* gb, int act, int B, int C, int L, int K, float* ws, hipStream_t st) {
+  using ET = typename Elem<DT>::T;
+  const int nparts = int(mma_runs(B, C, L)), run = int(mma_run_tiles(B, C, L));
+  const dim3 grid(C, unsigned(nparts));
+  const bool al = rows16<DT>(L, x, gy, gx);
+  with_band(K, [&](auto s) {
+    auto go = [&](auto a, auto f) {
+      hipLaunchKernelGGL((cconv_bwd_mma_kernel<DT, decltype(s)::value, decltype(f)::value, decltype(a)::value>), grid,
+                         dim3(kConvThreads), 0, st, (const ET*)gy, (const ET*)x, w, bias, (ET*)gx, ws, B, C, L, K,
+                         run);
+    };
+    using SILU = std::integral_constant<int, NSQ_ACT_SILU>;
+    using IDN = std::integral_constant<int, NSQ_ACT_IDENTITY>;
+    if (al)
+      act == NSQ_ACT_SILU ? go(std::true_type{}, SILU{}) : go(std::true_type{}, IDN{});
+    else
+      act == NSQ_ACT_SILU ? go(std::false_type{}, SILU{}) : go(std::false_type{}, IDN{});
+  });
+  hipLaunchKernelGGL(cconv_wgrad_reduce_kernel, dim3(C), dim3(kConvThreads + 64), 0, st, (const float*)ws, nparts, K,
+                     gw, gb);
+}
+
 // ---------------------------------------------------------------------------
-// Backward for K <= 16 taps in one register-resident pass (the Hyena
+// Backward for up to 8 taps (short_bwd) in one register-resident pass (the Hyena
 // short-conv case).  Thread t of a tile owns outputs n = n0 + 8t + e, e < 8.
-// With the taps left-padded to KP = 4, 8 or 16 (wk[j] = w[j - (KP - K)]):
+// With the taps left-padded to KP = 4 or 8 (wk[j] = w[j - (KP - K)]):
 //   pre[n]  = bias + sum_j wk[j] x[n - KP + 1 + j],  gpre = gy * silu'(pre) (or gy)
 //   gx[n]   = sum_s wr[s] gpre[n + s],                wr[s] = w[K - 1 - s] (s < K)
 //   gwk[j] += gpre[n] x[n - KP + 1 + j],              gb += gpre[n]
@@ -305,7 +517,7 @@ __global__ __launch_bounds__(kConvThreads) void cconv_bwd_short_kernel(
     const typename Elem<DT>::T* __restrict__ gy, const typename Elem<DT>::T* __restrict__ x,
     const float* __restrict__ w, const float* __restrict__ bias, typename Elem<DT>::T* __restrict__ gx,
     float* __restrict__ part, int B, int C, int L, int K) {
-  static_assert(KP == 4 || KP == 8 || KP == 16, "cconv_bwd_short: taps padded to 4, 8 or 16");
+  static_assert(KP == 4 || KP == 8, "cconv_bwd_short: taps padded to 4 or 8");
   static_assert(kConvPer == 8, "cconv_bwd_short: 8 outputs per thread");
   constexpr int NG = kConvPer + KP - 1;  // gpre positions per thread: [0, NG)
   constexpr int XB = (KP - 1 + 7) / 8;   // x chunks before the outputs: positions >= 1 - KP
@@ -387,19 +599,15 @@ static void launch_bwd_short(const void* gy, const void* x, const float* w, cons
   using ET = typename Elem<DT>::T;
   const int64_t nparts = cconv_wgrad_parts(B, L);
   dim3 grid(C, unsigned(nparts));
-  const bool al = L % (DT == NSQ_DTYPE_F32 ? 4 : 8) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-                  (reinterpret_cast<uintptr_t>(gy) & 15) == 0 && (reinterpret_cast<uintptr_t>(gx) & 15) == 0;
+  const bool al = rows16<DT>(L, x, gy, gx);
   auto go = [&](auto al_c, auto act_c) {
     constexpr bool A = decltype(al_c)::value;
     constexpr int F = decltype(act_c)::value;
     if (K <= 4)
       hipLaunchKernelGGL((cconv_bwd_short_kernel<DT, A, F, 4>), grid, dim3(kConvThreads), 0, st, (const ET*)gy,
                          (const ET*)x, w, bias, (ET*)gx, ws, B, C, L, K);
-    else if (K <= 8)
+    else if constexpr (A && DT == NSQ_DTYPE_F32)
       hipLaunchKernelGGL((cconv_bwd_short_kernel<DT, A, F, 8>), grid, dim3(kConvThreads), 0, st, (const ET*)gy,
-                         (const ET*)x, w, bias, (ET*)gx, ws, B, C, L, K);
-    else
-      hipLaunchKernelGGL((cconv_bwd_short_kernel<DT, A, F, 16>), grid, dim3(kConvThreads), 0, st, (const ET*)gy,
                          (const ET*)x, w, bias, (ET*)gx, ws, B, C, L, K);
   };
   using T_ = std::true_type;
@@ -418,29 +626,23 @@ template <int DT>
 static void launch_fwd(const void* x, const float* w, const float* bias, void* y, int act, int B, int C, int L, int K,
                        hipStream_t st) {
   using ET = typename Elem<DT>::T;
-  if (K > 16) {  // matrix cores; up to 16 taps the register kernel below is faster
-    switch (mfma_steps_for(K)) {  // 17 <= K <= 256 (validated)
-      case 12: return launch_fwd_mfma<DT, 12>(x, w, bias, y, act, B, C, L, K, st);
-      case 20: return launch_fwd_mfma<DT, 20>(x, w, bias, y, act, B, C, L, K, st);
-      case 36: return launch_fwd_mfma<DT, 36>(x, w, bias, y, act, B, C, L, K, st);
-      default: return launch_fwd_mfma<DT, 68>(x, w, bias, y, act, B, C, L, K, st);
-    }
-  }
+  const bool al = rows16<DT>(L, x, y, nullptr);
+  if (!short_fwd<DT>(K, act, int64_t(B) * C * L, al)) return launch_fwd_mma<DT>(x, w, bias, y, act, B, C, L, K, st);
   dim3 grid(B * C, unsigned(ceil_div(L, kConvTile)));
-  const bool al = L % (DT == NSQ_DTYPE_F32 ? 4 : 8) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-                  (reinterpret_cast<uintptr_t>(y) & 15) == 0;
   auto go = [&](auto al_c, auto act_c) {
     constexpr bool A = decltype(al_c)::value;
     constexpr int F = decltype(act_c)::value;
     if (K <= 4)
       hipLaunchKernelGGL((cconv_fwd_short_kernel<DT, A, F, 4>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
                          bias, (ET*)y, C, L, K);
-    else if (K <= 8)
-      hipLaunchKernelGGL((cconv_fwd_short_kernel<DT, A, F, 8>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
-                         bias, (ET*)y, C, L, K);
-    else
-      hipLaunchKernelGGL((cconv_fwd_short_kernel<DT, A, F, 16>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
-                         bias, (ET*)y, C, L, K);
+    else if constexpr (A || (DT != NSQ_DTYPE_F32 && F == NSQ_ACT_IDENTITY)) {
+      if (K <= 8)
+        hipLaunchKernelGGL((cconv_fwd_short_kernel<DT, A, F, 8>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
+                           bias, (ET*)y, C, L, K);
+      else if constexpr (A && DT == NSQ_DTYPE_F32)
+        hipLaunchKernelGGL((cconv_fwd_short_kernel<DT, A, F, 16>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
+                           bias, (ET*)y, C, L, K);
+    }
   };
   using T_ = std::true_type;
   using F_ = std::false_type;
@@ -455,13 +657,9 @@ static void launch_fwd(const void* x, const float* w, const float* bias, void* y
 template <int DT>
 static void launch_bwd(const void* gy, const void* x, const float* w, const float* bias, void* gx, float* gw,
                        float* gb, int act, int B, int C, int L, int K, float* ws, hipStream_t st) {
-  if (K <= 16) return launch_bwd_short<DT>(gy, x, w, bias, gx, gw, gb, act, B, C, L, K, ws, st);
-  switch (mfma_steps_for(K)) {  // 17 <= K <= 256 (validated)
-    case 12: return launch_bwd_mfma<DT, 12>(gy, x, w, bias, gx, gw, gb, act, B, C, L, K, ws, st);
-    case 20: return launch_bwd_mfma<DT, 20>(gy, x, w, bias, gx, gw, gb, act, B, C, L, K, ws, st);
-    case 36: return launch_bwd_mfma<DT, 36>(gy, x, w, bias, gx, gw, gb, act, B, C, L, K, ws, st);
-    default: return launch_bwd_mfma<DT, 68>(gy, x, w, bias, gx, gw, gb, act, B, C, L, K, ws, st);
-  }
+  if (short_bwd<DT>(K, int64_t(B) * C * L, rows16<DT>(L, x, gy, gx)))
+    return launch_bwd_short<DT>(gy, x, w, bias, gx, gw, gb, act, B, C, L, K, ws, st);
+  launch_bwd_mma<DT>(gy, x, w, bias, gx, gw, gb, act, B, C, L, K, ws, st);
 }
 
 static int validate_cconv(const void* a, const void* b, const float* w, int dtype, int act, int64_t B, int64_t C,
@@ -504,6 +702,16 @@ static float* noalloc_scratch() {
   return g_scratch[dev];
 }
 
+// What the noalloc entry point counts against its scratch, which fixes the shapes it takes: partials of one run per
+// kConvSegTiles tiles, and for silu above 16 taps an fp32 row set [B, C, L].  Never less than the backward
+// uses where that fits (at most max(C, kMmaTarget + C) partial rows).
+static size_t noalloc_bytes(int64_t B, int64_t C, int64_t L, int64_t K, int act) {
+  const int64_t pre = act == NSQ_ACT_SILU && K > 16 ? B * C * L : 0;
+  const size_t was = size_t(pre + C * cconv_wgrad_parts(B, L) * (K + 1)) * sizeof(float);
+  const size_t now = nsq_causal_conv1d_bwd_workspace_bytes(B, C, L, K, act);
+  return was > now ? was : now;
+}
+
 template <class... A>
 static void launch_bwd_dtype(int dtype, A... a) {
   switch (dtype) {
@@ -520,13 +728,11 @@ using namespace nsq;
 extern "C" {
 
 size_t nsq_causal_conv1d_bwd_workspace_bytes(int64_t B, int64_t C, int64_t L, int64_t K, int activation) {
-  // K <= 16 (one fused pass): the weight / bias gradient partials
-  // [C][parts][K + 1] only; otherwise (matrix cores) silu: gy * silu'(pre)
-  // [B, C, L], then the partials
-  if (K >= 1 && K <= 16) return size_t(C * cconv_wgrad_parts(B, L) * (K + 1)) * sizeof(float);
-  const int64_t pre = activation == NSQ_ACT_SILU ? B * C * L : 0;
-  const int64_t parts = K <= kConvMaxK ? C * cconv_wgrad_parts(B, L) * (K + 1) : 0;
-  return size_t(pre + parts) * sizeof(float);
+  (void)activation;
+  // the weight / bias gradient partials [C][parts][K + 1]
+  if (K < 1 || K > kConvMaxK || B < 1 || C < 1 || L < 1) return 0;
+  const int64_t few = cconv_wgrad_parts(B, L), runs = mma_runs(B, C, L), parts = few > runs ? few : runs;
+  return size_t(C * parts * (K + 1)) * sizeof(float);
 }
 
 int nsq_causal_conv1d_fwd(const void* x, const float* weight, const float* bias, void* y, int dtype, int activation,
@@ -570,7 +776,7 @@ int nsq_causal_conv1d_bwd_noalloc(const void* gy, const void* x, const float* we
   int rc = validate_cconv(gy, x, weight, dtype, activation, B, C, L, K);
   if (rc) return rc;
   NSQ_CHECK_ARG(gx && gweight, "causal_conv1d_bwd_noalloc: null gradient output pointer");
-  const size_t need = nsq_causal_conv1d_bwd_workspace_bytes(B, C, L, K, activation);
+  const size_t need = noalloc_bytes(B, C, L, K, activation);
   if (need > kNoAllocScratchBytes) {
     set_error("causal_conv1d_bwd_noalloc: B=%lld C=%lld L=%lld K=%lld needs %zu bytes of scratch, more than the "
               "fixed %zu-byte device buffer; call nsq_causal_conv1d_bwd with a workspace instead",

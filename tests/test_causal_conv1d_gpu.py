@@ -338,3 +338,35 @@ def test_b2b_16bit_io_mixer_as_bf16_products(dtype, tol, Km):
     assert rel_l2(y64, y) < tol
     assert rel_l2(y64[..., :Km + 3], y[..., :Km + 3]) < tol
     assert rel_l2(y64[..., 2048:2048 + Km], y[..., 2048:2048 + Km]) < tol
+
+
+@pytest.mark.parametrize("act", ["identity", "silu"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,C,L,K", [(1, 2048, 6 * 2048 + 8, 18), (1, 2048, 5 * 2048, 145), (3, 70, 4100, 210),
+                                     (2, 1, 2049, 256), (1, 3, 255, 17), (2, 5, 2047, 81)])
+def test_bands_as_split_bf16_products(B, C, L, K, dtype, act):
+    """The matrix-core bands (operands as exact sums of bf16 values) against float64 of the same inputs: tap counts at
+    the step boundaries, runs of tiles that start inside a row (2048 channels: three or five tiles a run) or span
+    rows, one-sample tails, unaligned rows.  fp32 values (weight and bias gradients in every type) are sums of up to
+    B L products: 1e-6 relative, a few fp32 roundings; 16-bit outputs are one rounding, half a unit in the last
+    place at most 2^-9 / 2^-12 relative.  A weight or bias gradient is a sum of B L terms of unit size, typically
+    sqrt(B L) and where it cancels (one channel's bias) anything below, while its rounding error follows the terms:
+    those errors are taken relative to sqrt(B L) per entry where that is more."""
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(B, C, L, device="cuda", generator=gen).to(dtype).requires_grad_()
+    gy = torch.randn(B, C, L, device="cuda", generator=gen).to(dtype)
+    w = (torch.randn(C, K, device="cuda", generator=gen) / K ** 0.5).requires_grad_()
+    b = torch.randn(C, device="cuda", generator=gen).requires_grad_()
+    y = causal_conv1d(x, w, b, act)
+    got = (y, *torch.autograd.grad(y, (x, w, b), gy))
+
+    x6, w6, b6 = (t.detach().double().requires_grad_() for t in (x, w, b))
+    n = L + K
+    p = torch.fft.irfft(torch.fft.rfft(x6, n=n) * torch.fft.rfft(w6.flip(-1), n=n), n=n)[..., :L] + b6.view(1, C, 1)
+    y6 = p * torch.sigmoid(p) if act == "silu" else p
+    want = (y6, *torch.autograd.grad(y6, (x6, w6, b6), gy.double()))
+    tol = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]
+    for i, (a, r) in enumerate(zip(got, want)):
+        size = r.norm().item() if i < 2 else max(r.norm().item(), (r.numel() * B * L) ** 0.5)
+        err = (a.double() - r).norm().item() / size
+        assert err < (tol if i < 2 else 1e-6), (i, err)
