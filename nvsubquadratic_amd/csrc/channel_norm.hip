@@ -421,26 +421,32 @@ __global__ __launch_bounds__(kThreads) void chnorm_bwd_kernel(
     for (int c = t; c < C; c += kThreads) db_part[wg * C + c] = gaccb[c];
 }
 
-// dw[c] = sum over the partial rows: a workgroup takes 64 channels, its four
-// lane groups rows r = 4k + q (q = 0..3, four running sums each over r mod 16),
-// combined in a fixed order (deterministic).
+// dw[c] = sum over the partial rows: a workgroup takes 16 channels (64-byte
+// pieces of a row), its 16 lane groups rows r = 16 k + q (four running sums
+// each), combined in a fixed order (deterministic).  Few channels mean few
+// workgroups: 512 rows of 384 took 15 us with 64 channels a workgroup.
 __global__ __launch_bounds__(kThreads) void chnorm_dw_reduce_kernel(const float* __restrict__ part,
                                                                     float* __restrict__ dw, int C, int64_t rows) {
-  __shared__ float acc[4][64];
-  const int t = threadIdx.x, q = t / 64;
-  const int64_t c = int64_t(blockIdx.x) * 64 + (t % 64);
+  __shared__ float acc[16][16];
+  const int t = threadIdx.x, q = t / 16;
+  const int64_t c = int64_t(blockIdx.x) * 16 + (t % 16);
   float a[4] = {0.f, 0.f, 0.f, 0.f};
   if (c < C) {
     int64_t r = q;
-    for (; r + 12 < rows; r += 16) {
+    for (; r + 48 < rows; r += 64) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) a[j] += part[(r + 4 * j) * C + c];
+      for (int j = 0; j < 4; ++j) a[j] += part[(r + 16 * j) * C + c];
     }
-    for (; r < rows; r += 4) a[0] += part[r * C + c];
+    for (; r < rows; r += 16) a[0] += part[r * C + c];
   }
-  acc[q][t % 64] = (a[0] + a[1]) + (a[2] + a[3]);
+  acc[q][t % 16] = (a[0] + a[1]) + (a[2] + a[3]);
   __syncthreads();
-  if (q == 0 && c < C) dw[c] = (acc[0][t] + acc[1][t]) + (acc[2][t] + acc[3][t]);
+  if (q == 0 && c < C) {
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) s += acc[k][t];
+    dw[c] = s;
+  }
 }
 
 size_t fwd_lds(int C, int TS, int VW) { return (size_t(C) * (TS + 1) + size_t(kThreads) * VW + TS) * 4; }
@@ -487,6 +493,14 @@ void allow_lds(K* kernel, size_t lds) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                               int(lds));
 }
+}  // namespace
+}  // namespace nsq
+
+#include "channel_norm16.h"
+
+namespace nsq {
+namespace {
+
 // The kernels take the norm as a template argument.
 template <class F>
 void with_mode(int mode, F&& f) {
@@ -496,6 +510,26 @@ void with_mode(int mode, F&& f) {
     f(std::integral_constant<int, CHN_L2>{});
   else
     f(std::integral_constant<int, CHN_RMS>{});
+}
+// The register kernels of 16-bit tensors (channel_norm16.h): whole aligned 16-byte runs, C up to kNorm16MaxC,
+// offsets within a batch row in 32 bits.
+template <int DT>
+bool norm16_ok(int C, int64_t S, std::initializer_list<const void*> ptrs) {
+  return DT != NSQ_DTYPE_F32 && C <= kNorm16MaxC && C * S < (int64_t(1) << 30) && use_vec(8, C, S, 8, ptrs);
+}
+template <int DT, bool BWD, class F>
+void with_norm16_kernel(int C, bool gated, int act, int mode, F&& f) {
+  if constexpr (DT != NSQ_DTYPE_F32)
+    with_norm16<BWD>(C, [&](auto cfg) {
+      with_mode(mode, [&](auto mc) {
+        if (!gated) return f(cfg, mc, std::integral_constant<int, kNoGate>{});
+        if constexpr (decltype(mc)::value != CHN_L2) {  // the L2 norm has no gate
+          if (act == NSQ_GATE_SIGMOID) return f(cfg, mc, std::integral_constant<int, NSQ_GATE_SIGMOID>{});
+          if (act == NSQ_GATE_SILU) return f(cfg, mc, std::integral_constant<int, NSQ_GATE_SILU>{});
+          return f(cfg, mc, std::integral_constant<int, NSQ_GATE_IDENTITY>{});
+        }
+      });
+    });
 }
 template <int DT, int VW>
 void launch_fwd_vw(const void* y, const void* v, const float* w, const float* bias, void* out, int64_t B, int C,
@@ -514,6 +548,19 @@ template <int DT>
 void launch_fwd(const void* y, const void* v, const float* w, void* out, int64_t B, int C, int64_t S, float eps,
                 int gated, int act, int out_blh, hipStream_t st, int mode = CHN_RMS, const float* bias = nullptr) {
   constexpr int VW = 16 / int(sizeof(typename Elem<DT>::T));
+  if (norm16_ok<DT>(C, S, {y, v, out})) {
+    with_norm16_kernel<DT, false>(C, gated, act, mode, [&](auto cfg, auto mc, auto gt) {
+      using T = typename Elem<DT>::T;
+      using F = decltype(cfg);
+      auto* k = &chnorm16_fwd_kernel<DT, decltype(mc)::value, decltype(gt)::value, F>;
+      const int64_t tpb = ceil_div(S, int64_t(F::TS)), nt = B * tpb;
+      const size_t lds = norm16_lds<F>(C, 1);
+      allow_lds(k, lds);
+      hipLaunchKernelGGL(k, dim3(unsigned(nt)), dim3(F::NT), lds, st, (const T*)y, (const T*)v, w, bias, (T*)out, C,
+                         S, tpb, nt, eps, out_blh);
+    });
+    return;
+  }
   const int TS = pick_ts(C, false);
   if (use_vec(VW, C, S, TS, {y, v, out}))
     launch_fwd_vw<DT, VW>(y, v, w, bias, out, B, C, S, TS, eps, gated, act, out_blh, mode, st);
@@ -539,17 +586,34 @@ template <int DT>
 void launch_bwd(const void* dout, const void* y, const void* v, const float* w, void* dy, void* dv, float* dw,
                 float* part, const BwdPlan& p, int64_t B, int C, int64_t S, float eps, int gated, int act,
                 int out_blh, hipStream_t st, int mode = CHN_RMS, float* db = nullptr) {
-  (void)B;
   constexpr int VW = 16 / int(sizeof(typename Elem<DT>::T));
   float* partb = (mode == CHN_LN && db) ? part + p.nwg * int64_t(C) : nullptr;
-  if (use_vec(VW, C, S, p.TS, {dout, y, v, dy, dv}))
+  int64_t nwg = p.nwg;
+  // above 1024 channels a lane's vectors spill: a few tiles run no faster than the tile kernel (C = 1536, 784
+  // positions: 77 / 70 us; 25088: 249 / 748)
+  if (norm16_ok<DT>(C, S, {dout, y, v, dy, dv}) && (C <= 1024 || B * S >= 4096)) {
+    with_norm16_kernel<DT, true>(C, gated, act, mode, [&](auto cfg, auto mc, auto gt) {
+      using T = typename Elem<DT>::T;
+      using F = decltype(cfg);
+      auto* k = &chnorm16_bwd_kernel<DT, decltype(mc)::value, decltype(gt)::value, F>;
+      const int64_t tpb = ceil_div(S, int64_t(F::TS)), nt = B * tpb;
+      // one resident round: two 512-thread workgroups a CU or one of 1024; no more rows of partials than planned
+      nwg = nt < 512 * 512 / F::NT ? nt : 512 * 512 / F::NT;
+      if (nwg >= 8) nwg -= nwg % 8;
+      if (nwg > p.nwg) nwg = p.nwg;
+      const size_t lds = norm16_lds<F>(C, 3);
+      allow_lds(k, lds);
+      hipLaunchKernelGGL(k, dim3(unsigned(nwg)), dim3(F::NT), lds, st, (const T*)dout, (const T*)y, (const T*)v, w,
+                         (T*)dy, (T*)dv, dw ? part : nullptr, partb, C, S, tpb, nt, eps, out_blh);
+    });
+  } else if (use_vec(VW, C, S, p.TS, {dout, y, v, dy, dv}))
     launch_bwd_vw<DT, VW>(dout, y, v, w, dy, dv, part, partb, p, C, S, eps, gated, act, out_blh, mode, st);
   else
     launch_bwd_vw<DT, 1>(dout, y, v, w, dy, dv, part, partb, p, C, S, eps, gated, act, out_blh, mode, st);
-  const dim3 rgrid(unsigned(ceil_div(int64_t(C), int64_t(64))));
-  if (dw) hipLaunchKernelGGL(chnorm_dw_reduce_kernel, rgrid, dim3(kThreads), 0, st, (const float*)part, dw, C, p.nwg);
+  const dim3 rgrid(unsigned(ceil_div(int64_t(C), int64_t(16))));
+  if (dw) hipLaunchKernelGGL(chnorm_dw_reduce_kernel, rgrid, dim3(kThreads), 0, st, (const float*)part, dw, C, nwg);
   if (partb)
-    hipLaunchKernelGGL(chnorm_dw_reduce_kernel, rgrid, dim3(kThreads), 0, st, (const float*)partb, db, C, p.nwg);
+    hipLaunchKernelGGL(chnorm_dw_reduce_kernel, rgrid, dim3(kThreads), 0, st, (const float*)partb, db, C, nwg);
 }
 int check_common(const char* who, int dtype, int64_t B, int C, int64_t S, float eps, int gated, int act) {
   NSQ_CHECK_ARG(dtype == NSQ_DTYPE_F32 || dtype == NSQ_DTYPE_BF16 || dtype == NSQ_DTYPE_F16, "%s: bad dtype %d", who,

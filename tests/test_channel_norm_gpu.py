@@ -441,3 +441,32 @@ def test_groupnorm_opcheck():
     b = torch.rand(16, device="cuda", requires_grad=True)
     torch.library.opcheck(N.gated_channel_groupnorm_op, (y, v, w, b, 4, 1e-5, 2))
     torch.library.opcheck(N.gated_channel_groupnorm_op, (y, None, None, None, 1, 1e-5, 0))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,C,S", [(1, 8, 8), (2, 64, 72), (1, 72, 1000), (2, 136, 40), (1, 192, 24), (3, 264, 104),
+                                   (1, 392, 40), (1, 520, 72), (1, 776, 40), (2, 1032, 2056), (1, 1536, 4104)])
+def test_16bit_register_kernels(B, C, S, dtype):
+    """Whole 16-byte runs with C at the edges of the register kernels' configurations (blocks of 16 channels over 4, 8
+    or 16 waves) and a partial last tile, several tiles a workgroup at the larger ones: RMS in both layouts against the
+    CPU oracle, LayerNorm and L2 against the same sequence in float64 (u rounded to the I/O type as the gate rounds).
+    Tolerances as everywhere here: one or two roundings to the I/O type per value."""
+    _case(B, C, (S,), dtype, "sigmoid", True, seed=C)
+    _case(B, C, (S,), dtype, None, False, seed=C + 1)
+    gen = torch.Generator(device="cuda").manual_seed(C)
+    y, v, go = (torch.randn(B, C, S, device="cuda", generator=gen).to(dtype) for _ in range(3))
+    w, b = torch.randn(C, device="cuda", generator=gen), torch.randn(C, device="cuda", generator=gen)
+    args = [t.clone().requires_grad_() for t in (y, v, w, b)]
+    out = N.gated_channel_layernorm(*args, 1e-5, "silu", channels_last_out=False)
+    got = (out, *torch.autograd.grad(out, args, go))
+    y6, v6, w6, b6 = (t.double().requires_grad_() for t in (y, v, w, b))
+    ref = torch.nn.functional.layer_norm((y6 * torch.nn.functional.silu(v6)).movedim(1, -1), (C,), w6, b6, 1e-5).movedim(-1, 1)
+    for i, (r, o) in enumerate(zip((ref, *torch.autograd.grad(ref, (y6, v6, w6, b6), go.double())), got)):
+        assert rel_l2(r, o) < TOL[dtype], i
+    x = y.clone().requires_grad_()
+    out = N.channel_l2norm(x, 1e-6, True)
+    gx, = torch.autograd.grad(out, x, go.movedim(1, -1).contiguous())
+    x6 = y.double().requires_grad_()
+    ref = torch.nn.functional.normalize(x6, dim=1, eps=1e-6)
+    assert rel_l2(ref.movedim(1, -1), out) < TOL[dtype]
+    assert rel_l2(torch.autograd.grad(ref, x6, go.double())[0], gx) < TOL[dtype]
