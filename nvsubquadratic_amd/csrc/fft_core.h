@@ -255,8 +255,8 @@ struct TwTable {
 // of a pass waits, in issue order, behind the tile's HBM loads and stores, so
 // 4 loads and 11 complex products per radix-16 butterfly instead of 15 loads
 // take ~10% off the 4-step row kernels, whose VALU is far from busy.
-template <int R>
-__device__ __forceinline__ void pass_twiddles(const TwTable& tt, int seg, int k, float2* w) {
+template <int R, class TT>
+__device__ __forceinline__ void pass_twiddles(const TT& tt, int seg, int k, float2* w) {
   w[1] = tt.load(seg, k);
   if constexpr (R >= 4) {
     w[2] = tt.load(seg, 2 * k);

@@ -1,0 +1,6 @@
+// bf16 instances of the small-plane 2D convolution.
+#include "fftconv2d_plane_impl.h"
+
+namespace nsq {
+NSQ_PLANE2_INSTANCES(NSQ_DTYPE_BF16)
+}  // namespace nsq

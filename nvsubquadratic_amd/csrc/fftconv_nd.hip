@@ -19,6 +19,12 @@ int nd_fwd(int nd, const void* x, const float* k, const void* shortcut, void* y,
   hipStream_t st = (hipStream_t)stream;
   float2* ws = (float2*)workspace;
   const bool save = workspace_bytes >= nd_workspace_bytes(nd, B, H, S, K, kbatch, periodic, NSQ_DIR_BWD);
+  Plane2Size z;
+  if (plane2_size(p, z)) {  // keeps no state: its backward transforms x and k again, in LDS
+    plane2_fwd(dtype, p, z, x, k, shortcut, y, nullptr, tw, st);
+    NSQ_CHECK_LAUNCH();
+    return NSQ_OK;
+  }
   bool ok;
   switch (dtype) {
     case NSQ_DTYPE_F32: ok = run_nd_fwd<NSQ_DTYPE_F32>(p, x, k, shortcut, y, ws, save, tw, st); break;
@@ -46,6 +52,12 @@ int nd_bwd(int nd, const void* g, const void* x, const float* k, const void* sho
   if (!tw) return NSQ_ERR_HIP;
   hipStream_t st = (hipStream_t)stream;
   float2* ws = (float2*)workspace;
+  Plane2Size z;
+  if (plane2_size(p, z)) {
+    plane2_bwd(dtype, p, z, g, x, k, shortcut, gx, gk, gs, ws, nullptr, tw, st);
+    NSQ_CHECK_LAUNCH();
+    return NSQ_OK;
+  }
   bool ok;
   switch (dtype) {
     case NSQ_DTYPE_F32: ok = run_nd_bwd<NSQ_DTYPE_F32>(p, g, x, k, shortcut, gx, gk, gs, ws, fwd_state != 0, tw, st); break;

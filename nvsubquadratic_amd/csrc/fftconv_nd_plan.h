@@ -703,6 +703,57 @@ NSQ_ND_RUN_INSTANCES(extern, NSQ_DTYPE_F32, true)
 NSQ_ND_RUN_INSTANCES(extern, NSQ_DTYPE_BF16, true)
 NSQ_ND_RUN_INSTANCES(extern, NSQ_DTYPE_F16, true)
 
+// Small planes with whole images in LDS (fftconv2d_plane_*.hip): transform lengths 2^lF0 and 2^(lM + 1).
+struct Plane2Size {
+  int lF0, lM;
+};
+// The plane of a plan's shape, if this path takes it: zero-padded last axis, axis 0 zero-padded or periodic of at
+// least 16 points, transform lengths (the powers of two that hold the linear extent) of at most 128.  Where the
+// mixed-radix plan takes 96 x 96 the 128 x 128 plane (1024 threads, spills in the adjoint) is no faster (B=16 H=256
+// 48 x 48: 381 / 367 us forward + backward); every smaller plane is (24 x 24, 64 x 64 against 48 x 48: 60 / 95).
+inline bool plane2_size(const NdPlan& p, Plane2Size& z) {
+  if (p.nd != 2 || p.r[2] != 0 || p.wm[0] != -1 || p.wm[2] != -1) return false;
+  if (p.o[2] == 0 && p.F[2] == p.S[2]) return false;  // periodic, one tap
+  const bool per0 = p.o[0] == 0 && p.F[0] == p.S[0];
+  z.lF0 = per0 ? p.lF[0] : ilog2_ceil(int64_t(p.S[0]) + (p.K[0] + 1) / 2);
+  z.lM = ilog2_ceil(int64_t(p.S[2]) + (p.K[2] + 1) / 2) - 1;
+  if (z.lF0 < 4) z.lF0 = 4;
+  if (z.lM < 3) z.lM = 3;
+  if (z.lF0 + z.lM < 9) {  // at least one wave of 8 points a lane
+    if (per0)
+      z.lM = 9 - z.lF0;
+    else
+      z.lF0 = 9 - z.lM;
+  }
+  return z.lF0 <= 7 && z.lM <= 6 && !(p.r3 && z.lF0 + z.lM == 13);
+}
+// gate: the Hyena gates' operands (x is then q; gated_nd_fwd / gated_nd_bwd), or null.
+template <int DT>
+void plane2_fwd(const NdPlan& p, const Plane2Size& z, const void* x, const float* k, const void* s, void* y,
+                const GatedIO* gate, const float2* tw, hipStream_t st);
+template <int DT>
+void plane2_bwd(const NdPlan& p, const Plane2Size& z, const void* gy, const void* x, const float* k, const void* s,
+                void* gx, float* gk, float* gs, float* ws, const GatedIO* gate, const float2* tw, hipStream_t st);
+// By dtype code; ws: the backward's conv workspace (partial filter gradients).
+inline void plane2_fwd(int dtype, const NdPlan& p, const Plane2Size& z, const void* x, const float* k, const void* s,
+                       void* y, const GatedIO* gate, const float2* tw, hipStream_t st) {
+  switch (dtype) {
+    case NSQ_DTYPE_F32: return plane2_fwd<NSQ_DTYPE_F32>(p, z, x, k, s, y, gate, tw, st);
+    case NSQ_DTYPE_BF16: return plane2_fwd<NSQ_DTYPE_BF16>(p, z, x, k, s, y, gate, tw, st);
+    default: return plane2_fwd<NSQ_DTYPE_F16>(p, z, x, k, s, y, gate, tw, st);
+  }
+}
+inline void plane2_bwd(int dtype, const NdPlan& p, const Plane2Size& z, const void* gy, const void* x, const float* k,
+                       const void* s, void* gx, float* gk, float* gs, void* ws, const GatedIO* gate, const float2* tw,
+                       hipStream_t st) {
+  float* part = static_cast<float*>(ws);
+  switch (dtype) {
+    case NSQ_DTYPE_F32: return plane2_bwd<NSQ_DTYPE_F32>(p, z, gy, x, k, s, gx, gk, gs, part, gate, tw, st);
+    case NSQ_DTYPE_BF16: return plane2_bwd<NSQ_DTYPE_BF16>(p, z, gy, x, k, s, gx, gk, gs, part, gate, tw, st);
+    default: return plane2_bwd<NSQ_DTYPE_F16>(p, z, gy, x, k, s, gx, gk, gs, part, gate, tw, st);
+  }
+}
+
 // Plain and mixed-boundary conv (fftconv_nd.hip).
 int nd_fwd(int nd, const void* x, const float* k, const void* shortcut, void* y, int dtype, int64_t B, int64_t H,
            const int64_t* S, const int64_t* K, int64_t kbatch, unsigned periodic, void* workspace,
