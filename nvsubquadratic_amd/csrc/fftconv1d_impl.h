@@ -28,7 +28,7 @@
 #include <cstdlib>
 
 #include "fft_core.h"
-#include "gate.h"
+#include "fftconv1d_ring.h"
 
 namespace nsq {
 
@@ -254,68 +254,6 @@ __global__ __launch_bounds__(FusedCfg<LOGN>::T) void fused_fwd_kernel(
       __syncthreads();
     }
   }
-}
-
-// Forward, fused plan, for grids too small to fill the GPU (M == 1 lengths,
-// few (channel, batch row) pairs): fused_fwd_kernel then runs one workgroup
-// of N/16 threads per row, one wave per SIMD, and transforms the filter and
-// the row one after the other.  Here a workgroup of 2 N/2^LOGRMAX threads
-// owns one (channel h = blockIdx.x, batch row b = blockIdx.y) and holds a
-// two-transform tile: transform 0 is the filter, transform 1 the row, both
-// transformed at once (the first half of the threads load the filter, the
-// rest the row).  The product reads both spectra from LDS slot by slot and
-// leaves the result in transform 1; the inverse transform runs over the whole
-// tile and the epilogue keeps transform 1.  With LOGRMAX = 4 the arithmetic
-// per element is that of fused_fwd_kernel (bitwise equal outputs); LOGRMAX =
-// 3 runs radix-8 passes at 8 points per thread (agreement to fp32 rounding).
-// Plain causal conv (no fold, ramp or gates); kfilm: the filter row is image
-// b's.
-template <int LOGN, int DT, int LOGRMAX = 4>
-__global__ __launch_bounds__(2 * (FusedCfg<LOGN>::N >> LOGRMAX)) void fused_fwd_pair_kernel(
-    const typename Elem<DT>::T* __restrict__ x, const float* __restrict__ k,
-    const typename Elem<DT>::T* __restrict__ s, typename Elem<DT>::T* __restrict__ y, int H, int L, int K,
-    const float2* __restrict__ tw, int kfilm) {
-  using C = FusedCfg<LOGN>;
-  static_assert(C::M == 1, "fused_fwd_pair_kernel: one transform per channel");
-  constexpr int T = 2 * (C::N >> LOGRMAX), SL = C::N / 2 / T;  // threads; product slots per thread
-  static_assert(SL >= 1 && (C::N / 2) % T == 0, "fused_fwd_pair_kernel: slot split");
-  __shared__ float2 lds[2 * C::SP];
-  const int h = blockIdx.x, b = blockIdx.y;
-  const int64_t row = (int64_t(b) * H + h) * L;
-  const float* kr = k + (kfilm ? int64_t(b) * H + h : int64_t(h)) * K;
-
-  auto ld = [&](int m, int n) -> float2 {
-    if (m == 0) return load_pair<NSQ_DTYPE_F32>(kr, 2 * int64_t(n), K);
-    return load_pair<DT>(x + row, 2 * int64_t(n), L);
-  };
-  LdsTile<C::SP, true> st{lds};
-  fft_radix<LOGRMAX, LOGN, false, 2, T, C::SP>(lds, ld, st, tw);
-#pragma unroll
-  for (int i = 0; i < SL; ++i) {
-    NSQ_SLOT_FENCE();
-    const int p = opaque_tid() + i * T;
-    float2 hA, hB, A, Bc;
-    lds_unpack<LOGN>(lds, 0, p, tw, hA, hB);
-    lds_unpack<LOGN>(lds, 1, p, tw, A, Bc);
-    A = slot_mul(p == 0, A, hA);
-    Bc = cmul(Bc, hB);
-    lds_repack<LOGN>(lds, 1, p, tw, A, Bc);
-  }
-  __syncthreads();
-
-  const float scale = 1.f / float(C::N);
-  const float sv = s ? Elem<DT>::round(Elem<DT>::load(s, h)) : 0.f;
-  auto epi = [&](int m, int n, float2 v) {
-    if (m == 0) return;
-    const int64_t i0 = 2 * int64_t(n);
-    if (i0 < L)
-      Elem<DT>::store(y, row + i0, epilogue<DT>(v.x * scale, s != nullptr, sv, s ? Elem<DT>::load(x, row + i0) : 0.f));
-    if (i0 + 1 < L)
-      Elem<DT>::store(y, row + i0 + 1,
-                      epilogue<DT>(v.y * scale, s != nullptr, sv, s ? Elem<DT>::load(x, row + i0 + 1) : 0.f));
-  };
-  LdsTile<C::SP, true> ldl{lds};
-  fft_radix<LOGRMAX, LOGN, true, 2, T, C::SP>(lds, ldl, epi, tw);
 }
 
 // Backward, fused plan.  grid = ceil(H/M); each workgroup loops over all
@@ -1247,28 +1185,29 @@ __global__ __launch_bounds__(RowCfg<LOGN2>::T) __attribute__((amdgpu_waves_per_e
 // ===========================================================================
 // Host launchers
 // ===========================================================================
-// Largest B*H that the forward runs on fused_fwd_pair_kernel (M == 1 lengths,
-// no fold).  FFT length 16384 (radix-16 pair kernel): as many rows as one
-// round of pair workgroups covers, 256 CUs times the pair tiles that fit a
-// CU's 160 KB of LDS (256 rows; measured, one-transform -> pair kernel: H=256
-// 29.4 -> 23.2 us, H=512 39.4 -> 43.1 us).  FFT lengths 4096 and 8192
-// (radix-8 pair kernel): 1536 rows.  Measured at B=2 (kernel time, one-
-// transform -> pair kernel): length 8192, 256 rows 19.5 -> 13.5 us, 512 22.1
-// -> 20.0, 768 25.8 -> 26.3, 1024 38.4 -> 33.6, 1536 50.1 -> 48.5; length
-// 4096, 256 rows 16.2 -> 9.0 us, 1024 20.5 -> 17.8, 1536 25.7 -> 23.7, 2048
-// 28.7 -> 29.7.  NSQ_1D_PAIR_MAX_ROWS overrides the bound for every length (0
-// turns the pair kernel off).
+// Rule of the fused plan: lengths 1024..16384 without fold or shift run in the
+// ring z^F = -1 (fftconv1d_ring.h), at every grid size.  The others keep the
+// packed real transform: a folded transform has F < L + K - 1 and counts on
+// the ring z^F = 1, the circular one is defined by it, and below 1024 a
+// workgroup packs several channels into one tile.
 template <int LOGN>
-inline int64_t fused_pair_max_rows() {
-  static const int64_t env = [] {
-    const char* e = std::getenv("NSQ_1D_PAIR_MAX_ROWS");
-    return e ? int64_t(std::atoll(e)) : int64_t(-1);
-  }();
-  if (env >= 0) return env;
-  if constexpr (LOGN <= 12) return 1536;
-  constexpr int lds = 2 * FusedCfg<LOGN>::SP * int(sizeof(float2));
-  constexpr int per_cu = (160 * 1024) / lds;
-  return int64_t(256) * (per_cu < 1 ? 1 : per_cu);
+inline bool on_ring(const Plan1D& p) {
+  return LOGN >= 9 && !p.fold;
+}
+
+// The ring forward (fftconv1d_ring.h): a workgroup takes a second row of its channel only where the grid then still
+// has 2048 threads a CU.
+template <int LOGN, int DT, bool GATE>
+static void launch_ring_fwd(const void* x, const float* k, const void* s, void* y, int B, int H, int L, int K,
+                            int kfilm, const GateArgs& ga, const float2* tw, hipStream_t st) {
+  using ET = typename Elem<DT>::T;
+  constexpr int T = RingCfg<LOGN>::T, N = 1 << LOGN;
+  int nb = int(ceil_div(512 * 1024 / T, H));
+  nb = nb > B ? B : nb;
+  const int bpw = kfilm ? 1 : int(ceil_div(B, nb));
+  auto* kern = L > N || K > N ? &ring_fwd_kernel<LOGN, DT, true, GATE> : &ring_fwd_kernel<LOGN, DT, false, GATE>;
+  hipLaunchKernelGGL(kern, dim3(unsigned(H), unsigned(ceil_div(B, bpw))), dim3(T), 0, st, (const ET*)x, k,
+                     (const ET*)s, (ET*)y, B, H, L, K, bpw, tw, kfilm, ga);
 }
 
 // kfilm: per-sample filters [B*H, K]; one image per workgroup.
@@ -1277,15 +1216,8 @@ static void launch_fused_fwd(const Plan1D& p, const void* x, const float* k, con
                              int L, int K, int kfilm, const float2* tw, hipStream_t st) {
   using C = FusedCfg<LOGN>;
   using ET = typename Elem<DT>::T;
-  if constexpr (C::M == 1) {
-    if (!p.fold && int64_t(H) * B <= fused_pair_max_rows<LOGN>()) {
-      // radix-8 passes up to N = 4096 (2 N / 8 <= 1024 threads): twice the waves of the radix-16 form to cover
-      // the pass latencies of a grid of one round (FFT length 8192 at B=2 H=128: 17.6 -> 15.7 us per step)
-      constexpr int LOGR = LOGN <= 12 ? 3 : 4;
-      hipLaunchKernelGGL((fused_fwd_pair_kernel<LOGN, DT, LOGR>), dim3(H, B), dim3(2 * (C::N >> LOGR)), 0, st,
-                         (const ET*)x, k, (const ET*)s, (ET*)y, H, L, K, tw, kfilm);
-      return;
-    }
+  if constexpr (LOGN >= 9) {
+    if (on_ring<LOGN>(p)) return launch_ring_fwd<LOGN, DT, false>(x, k, s, y, B, H, L, K, kfilm, GateArgs{}, tw, st);
   }
   const int gh = int(ceil_div(H, C::M));
   int nb = int(ceil_div(2048, gh));
@@ -1296,7 +1228,7 @@ static void launch_fused_fwd(const Plan1D& p, const void* x, const float* k, con
   if (p.fold)
     hipLaunchKernelGGL((fused_fwd_kernel<LOGN, DT, true>), grid, dim3(C::T), 0, st, (const ET*)x, k, (const ET*)s,
                        (ET*)y, B, H, L, K, bpw, tw, 0, kfilm, -1, GateArgs{});
-  else
+  else if constexpr (LOGN < 9)
     hipLaunchKernelGGL((fused_fwd_kernel<LOGN, DT, false>), grid, dim3(C::T), 0, st, (const ET*)x, k, (const ET*)s,
                        (ET*)y, B, H, L, K, bpw, tw, 0, kfilm, -1, GateArgs{});
 }
@@ -1307,11 +1239,19 @@ static void launch_fused_bwd(const Plan1D& p, const void* g, const void* x, cons
                              hipStream_t st) {
   using C = FusedCfg<LOGN>;
   using ET = typename Elem<DT>::T;
+  if constexpr (LOGN >= 9) {
+    if (on_ring<LOGN>(p)) {
+      auto* kern = L > C::N || K > C::N ? &ring_bwd_kernel<LOGN, DT, true> : &ring_bwd_kernel<LOGN, DT, false>;
+      hipLaunchKernelGGL(kern, dim3(unsigned(H), unsigned(kfilm ? B : 1)), dim3(RingCfg<LOGN>::T), 0, st,
+                         (const ET*)g, (const ET*)x, k, (const ET*)s, (ET*)gx, gk, gs, B, H, L, K, tw, kfilm);
+      return;
+    }
+  }
   dim3 grid(unsigned(ceil_div(H, C::M)), unsigned(kfilm ? B : 1));
   if (p.fold)
     hipLaunchKernelGGL((fused_bwd_kernel<LOGN, DT, true>), grid, dim3(C::T), 0, st, (const ET*)g, (const ET*)x, k,
                        (const ET*)s, (ET*)gx, gk, gs, B, H, L, K, tw, 0, kfilm, -1, 1.f);
-  else
+  else if constexpr (LOGN < 9)
     hipLaunchKernelGGL((fused_bwd_kernel<LOGN, DT, false>), grid, dim3(C::T), 0, st, (const ET*)g, (const ET*)x, k,
                        (const ET*)s, (ET*)gx, gk, gs, B, H, L, K, tw, 0, kfilm, -1, 1.f);
 }
@@ -1323,6 +1263,9 @@ static void launch_gated_fused_fwd(const Plan1D& p, const void* q, const float* 
                                    hipStream_t st) {
   using C = FusedCfg<LOGN>;
   using ET = typename Elem<DT>::T;
+  if constexpr (LOGN >= 9) {
+    if (on_ring<LOGN>(p)) return launch_ring_fwd<LOGN, DT, true>(q, k, s, y, B, H, L, K, kfilm, ga, tw, st);
+  }
   const int gh = int(ceil_div(H, C::M));
   int nb = int(ceil_div(2048, gh));
   nb = nb < 1 ? 1 : (nb > B ? B : nb);
@@ -1332,7 +1275,7 @@ static void launch_gated_fused_fwd(const Plan1D& p, const void* q, const float* 
   if (p.fold)
     hipLaunchKernelGGL((fused_fwd_kernel<LOGN, DT, true, false, true>), grid, dim3(C::T), 0, st, (const ET*)q, k,
                        (const ET*)s, (ET*)y, B, H, L, K, bpw, tw, 0, kfilm, -1, ga);
-  else
+  else if constexpr (LOGN < 9)
     hipLaunchKernelGGL((fused_fwd_kernel<LOGN, DT, false, false, true>), grid, dim3(C::T), 0, st, (const ET*)q, k,
                        (const ET*)s, (ET*)y, B, H, L, K, bpw, tw, 0, kfilm, -1, ga);
 }
@@ -1763,10 +1706,10 @@ bool run_col_inv_rows(int logN, const float2* spec, float* out, float* gs, int64
 
 // Whether the fused plan's forward runs the gated kernel (gates in its first pass and epilogue) rather than the
 // gate kernels around the plain fused kernel.  Both round the same way (same bits).  The gated kernel adds four
-// operand streams (q and k in place of z, then q, k and v again in its epilogue, y1 beside y) to a kernel that
-// holds one or two workgroups per CU, so it only pays where launches dominate: measured on MI355X (bf16 fwd),
-// B=4 H=1024 L=8192 0.436 ms against 0.351 ms for the three kernels, B=1 H=1024 L=8192 0.110 / 0.100 ms,
-// B=2 H=256 L=4096 0.037 / 0.038 ms, B=1 H=64 L=2048 0.031 / 0.038 ms.  Below 2^22 elements the gated kernel;
+// operand streams (q and k in place of z, then q, k and v again in its epilogue, y1 beside y), single elements each, so
+// it only pays where launches dominate: measured on MI355X (bf16 fwd, us, three kernels / gated kernel), B=1 H=64
+// L=2048 13.6 / 11.7, B=2 H=256 L=4096 27 / 20, B=4 H=1024 L=1024 37 / 33, B=16 H=384 L=1000 46 / 46, B=4 H=1024
+// L=2048 59 / 63, B=1 H=1024 L=8192 81 / 101, B=4 H=1024 L=8192 251 / 340.  Below 2^22 elements the gated kernel;
 // NSQ_1D_GATES_FUSED=0 / 1 forces either.
 inline bool gates_fused_1d(const Plan1D& p, int64_t elems) {
   static const int force = [] {

@@ -496,3 +496,43 @@ def test_state_budget_zero_recomputes_bitwise(monkeypatch, L):
         grads.append([t.grad.clone() for t in (x, k, s)])
     for a, b in zip(*grads):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,L,K,film", [
+    (2, 3, 512, 512, False), (3, 2, 513, 7, True), (2, 2, 1000, 25, False),   # F = 1024: half, past it, L + K - 1 = F
+    (1, 2, 680, 345, False), (2, 3, 1025, 1024, False), (2, 2, 1024, 1025, True),  # F = 2048, each side past M
+    (3, 1, 2048, 2048, False), (1, 3, 3000, 1097, True), (2, 2, 4095, 4096, False), (2, 1, 8191, 2, True),
+    (2, 2, 8192, 8193, False), (1, 2, 16384, 1, False), (2, 1, 10923, 5462, False), (520, 1, 600, 40, False),
+])
+def test_fused_lengths_at_their_edges(B, H, L, K, film, dtype):
+    """Lengths 1024..16384 against float64, forward and gradients, with and without the shortcut.  The input values are
+    exact in `dtype`, so the fp32 results (filter and shortcut gradients, and everything in fp32) carry three
+    transforms of up to 14 stages: 3 * 14 * 2^-24 = 2.5e-6 relative to the full spectrum's norm, taken twice.  16-bit
+    outputs round the sum and the shortcut product: 2 * 2^-8 and 2 * 2^-11."""
+    torch.manual_seed(L + K)
+    x, g = (torch.randn(B, H, L).to(dtype) for _ in range(2))
+    k = torch.randn(B if film else 1, H, K) / K ** 0.5
+    s = torch.randn(H).to(dtype)
+    n = L + K
+    xf, kf, gf = (torch.fft.rfft(t.double(), n=n) for t in (x, k, g))
+    corr = torch.fft.irfft(gf * xf.conj(), n=n)[..., :K]
+    ref = {"y": torch.fft.irfft(xf * kf, n=n)[..., :L], "gx": torch.fft.irfft(gf * kf.conj(), n=n)[..., :L],
+           "gk": corr if film else corr.sum(0, keepdim=True)}
+    tol32 = 5e-6
+    tol = {torch.float32: tol32, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+    for shortcut in (False, True):
+        xd, kd = x.cuda().requires_grad_(True), k.cuda().requires_grad_(True)
+        sd = s.cuda().requires_grad_(True) if shortcut else None
+        y = F.causal_fftconv1d_bhl(xd, kd, sd)
+        y.backward(g.cuda())
+        sv = s.double()[:, None] if shortcut else 0.0
+        assert rel_l2(ref["y"] + sv * x.double(), y) < tol
+        assert rel_l2(ref["gx"] + sv * g.double(), xd.grad) < tol
+        # lags near K = L hold few samples: the error follows the whole row's spectrum, |g| |x| summed over images
+        full = sum(float(g[b].double().norm() * x[b].double().norm()) for b in range(B)) * (K / n) ** 0.5
+        assert (kd.grad.cpu().double() - ref["gk"]).norm() < tol32 * max(full, float(ref["gk"].norm()))
+        if shortcut:
+            gs = (g.double() * x.double()).sum((0, 2))
+            bound = (tol32 if dtype == torch.float32 else tol) * (g.double().norm() * x.double().norm())
+            assert (sd.grad.cpu().double() - gs).norm() < bound
