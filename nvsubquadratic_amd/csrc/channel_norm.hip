@@ -112,8 +112,10 @@ enum { CHN_RMS = 0, CHN_L2 = 1, CHN_LN = 2 };
 // Phase shared by both directions: u into U[c][s] (zero past S), per-position
 // r = rsqrt(mean u^2 + eps) (RMS), 1 / max(round(||u||), eps) (L2) or
 // rsqrt(mean (u - mu)^2 + eps) (LN, with U then holding u - mu) into rs[];
-// L2 with cl: cl[s] = 0 where the norm was clamped to eps, else 1.  red holds
-// G x TS partial sums.
+// L2 with cl: cl[s] = 0 where the norm was clamped to eps, else 1.  rs is 0
+// past S (u = 0 there, and with eps = 0 the formula gives inf, whose product
+// with u would reach the weight gradient as NaN).  red holds G x TS partial
+// sums.
 template <int DT, int VW>
 __device__ __forceinline__ void load_tile_u(const typename Elem<DT>::T* __restrict__ y,
                                             const typename Elem<DT>::T* __restrict__ v, bool gated, int act,
@@ -157,17 +159,18 @@ __device__ __forceinline__ void load_tile_u(const typename Elem<DT>::T* __restri
 #pragma unroll
   for (int k = 0; k < VW; ++k) red[m.g * TS + p0 + k] = ss[k];
   __syncthreads();
+  const bool inside = s0 + int(threadIdx.x) < S;
   if (threadIdx.x < TS) {
     float sum = 0.f;
     for (int k = 0; k < m.G; ++k) sum += red[k * TS + threadIdx.x];
     if (mode == CHN_L2) {
       const float n = Elem<DT>::round(sqrtf(sum));
-      rs[threadIdx.x] = 1.f / fmaxf(n, eps);
+      rs[threadIdx.x] = inside ? 1.f / fmaxf(n, eps) : 0.f;
       if (cl) cl[threadIdx.x] = n < eps ? 0.f : 1.f;
     } else if (mode == CHN_LN) {
       rs[threadIdx.x] = sum / float(C);  // the mean, until the second sweep
     } else {
-      rs[threadIdx.x] = rsqrtf(sum * (1.f / float(C)) + eps);
+      rs[threadIdx.x] = inside ? rsqrtf(sum * (1.f / float(C)) + eps) : 0.f;
     }
   }
   __syncthreads();
@@ -189,7 +192,7 @@ __device__ __forceinline__ void load_tile_u(const typename Elem<DT>::T* __restri
     if (threadIdx.x < TS) {
       float sum = 0.f;
       for (int k = 0; k < m.G; ++k) sum += red[k * TS + threadIdx.x];
-      rs[threadIdx.x] = rsqrtf(sum * (1.f / float(C)) + eps);
+      rs[threadIdx.x] = inside ? rsqrtf(sum * (1.f / float(C)) + eps) : 0.f;
     }
     __syncthreads();
   }

@@ -456,6 +456,7 @@ __global__ __launch_bounds__(F::NT) __attribute__((amdgpu_waves_per_eu(4))) void
       take8(tot + 32 * h + p0, r);
       take8(tot + F::TS + 32 * h + p0, m);
       if constexpr (MODE == CHN_LN) take8(tot + (K - 1) * F::TS + 32 * h + p0, mg);
+      const bool inside = 32 * h + p0 < nval;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         if constexpr (MODE == CHN_L2) {
@@ -467,6 +468,8 @@ __global__ __launch_bounds__(F::NT) __attribute__((amdgpu_waves_per_eu(4))) void
           m[k] = m[k] * r[k] * invC;
           if constexpr (MODE == CHN_LN) mg[k] *= invC;
         }
+        // past the tensor u = 0 and, at eps = 0, r = inf: their product would reach gw as NaN
+        if (!inside) r[k] = m[k] = 0.f;
       }
 #pragma unroll
       for (int j = 0; j < F::NB; ++j) {

@@ -470,3 +470,31 @@ def test_16bit_register_kernels(B, C, S, dtype):
     ref = torch.nn.functional.normalize(x6, dim=1, eps=1e-6)
     assert rel_l2(ref.movedim(1, -1), out) < TOL[dtype]
     assert rel_l2(torch.autograd.grad(ref, x6, go.double())[0], gx) < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("C,S", [(384, 40), (384, 784), (768, 784), (64, 72), (96, 33)])
+def test_zero_eps_with_a_partial_last_tile(C, S, dtype):
+    """eps = 0 is accepted: the positions a partial last tile holds past the tensor (u = 0, r = 1 / 0) stay out of the
+    weight gradients.  Every value of the inputs is finite and no column is zero, so every result is finite; compared
+    with the same sequence in float64 (one or two roundings to the I/O type per value)."""
+    print(f"C={C} S={S} {dtype}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(S)
+    y, v, go = (torch.randn(2, C, S, device="cuda", generator=gen).to(dtype) for _ in range(3))
+    w, b = 1 + 0.5 * torch.rand(C, device="cuda", generator=gen), torch.randn(C, device="cuda", generator=gen)
+    y6, v6, w6, b6 = (t.double().requires_grad_() for t in (y, v, w, b))
+
+    def rms6(y, v, w):
+        u = y * torch.sigmoid(v)
+        return w[:, None] * u * torch.rsqrt((u * u).mean(1, keepdim=True))
+
+    def ln6(y, v, w, b):
+        return torch.nn.functional.layer_norm((y * torch.sigmoid(v)).movedim(1, -1), (C,), w, b, 0.0).movedim(-1, 1)
+
+    for op, op6, n in ((N.gated_channel_rmsnorm, rms6, 3), (N.gated_channel_layernorm, ln6, 4)):
+        args, args6 = [t.clone().requires_grad_() for t in (y, v, w, b)[:n]], (y6, v6, w6, b6)[:n]
+        out, ref = op(*args, 0.0, "sigmoid", channels_last_out=False), op6(*args6)
+        got = (out, *torch.autograd.grad(out, args, go))
+        for i, (r, o) in enumerate(zip((ref, *torch.autograd.grad(ref, args6, go.double())), got)):
+            assert torch.isfinite(o).all(), i
+            assert rel_l2(r, o) < TOL[dtype], i
