@@ -113,6 +113,19 @@ static int64_t cconv_wgrad_parts(int64_t B, int64_t L) {
 // ---------------------------------------------------------------------------
 constexpr int kMmaTarget = 4096;  // workgroups wanted: 4 or more per resident slot (256 CUs x 2..4)
 
+// A band multiplies every sample of a block's window, later ones too, by some zero tap, and inf leaves NaN among its
+// parts (inf - inf; a finite value above the largest bf16 is inf in its first part): a non-finite value makes all the
+// sums over its window NaN.  So where all results are finite they are right, and where some are not the kernels take
+// the run's results once more at its end, tap by tap from memory.  (Not in place: that path's registers on top of the
+// bands' cost one to three waves per SIMD.  Checks of the operands, with flags in LDS, cost 5 to 10% of the time.)
+template <int N>
+__device__ __forceinline__ bool nonfinite(const float (&v)[N]) {
+  float s[2] = {0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < N; ++i) s[i & 1] = fmaf(v[i], 0.f, s[i & 1]);
+  return !(s[0] + s[1] == 0.f);
+}
+
 // Tiles per run: as many as leave kMmaTarget workgroups, at least 1.
 static int64_t mma_run_tiles(int64_t B, int64_t C, int64_t L) {
   const int64_t tiles = B * ceil_div(L, kConvTile), want = ceil_div(kMmaTarget, C);
@@ -188,6 +201,8 @@ cconv_fwd_mma_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __
   get_band<S>(band, tap);
   __syncthreads();
   const float b0 = bias ? bias[c] : 0.f;
+  const int p0 = 16 * (32 * wave + (l & 15)) + 4 * (l >> 4);  // the lane's positions in M-tile 2 wave; 256 on in the next
+  int bad = g1;  // the wave's first tile with a non-finite result
   for (int g = g0; g < g1; ++g) {
     const int b = g / ntiles, n0 = (g - b * ntiles) * kConvTile;
     uint16_t* xb = reinterpret_cast<uint16_t*>(sm + ((g - g0) & 1) * WIN);
@@ -206,12 +221,27 @@ cconv_fwd_mma_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __
     nsq_f32x4_t acc[2];
     band_run2<S, P>(tap, xb, W, 32 * wave, 32 * wave + 16, acc[0], acc[1]);
     const RowBuf<DT, false> ob(y + (int64_t(b) * C + c) * L, L);
+    float v[2][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[h][r] = acc[h][r] + b0;
+    if (__ballot(nonfinite(reinterpret_cast<const float(&)[8]>(v))) != 0) bad = min(bad, g);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      float v[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = act_fwd<ACT>(acc[h][r] + b0);
-      store4<DT, AL>(ob, n0 + 16 * (32 * wave + 16 * h + (l & 15)) + 4 * (l >> 4), v);
+      for (int r = 0; r < 4; ++r) v[h][r] = act_fwd<ACT>(v[h][r]);
+      store4<DT, AL>(ob, n0 + p0 + 256 * h, v[h]);
+    }
+  }
+#pragma unroll 1
+  for (int g = bad; g < g1; ++g) {  // each lane its own outputs
+    const int b = g / ntiles, n0 = (g - b * ntiles) * kConvTile;
+    const RowBuf<DT, false> rb(x + (int64_t(b) * C + c) * L, L), ob(y + (int64_t(b) * C + c) * L, L);
+#pragma unroll 1
+    for (int i = 0; i < 8; ++i) {
+      const int n = n0 + p0 + 256 * (i >> 2) + (i & 3);
+      if (n < L) ob.store_elem(n, act_fwd<ACT>(direct_taps<DT>(rb, w + int64_t(c) * K, K, n) + b0));
     }
   }
 }
@@ -226,7 +256,7 @@ cconv_fwd_mma_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __
 // LDS: both bands as operands (reloaded into registers per phase: together they would not fit beside D), the window
 // of x and gpre as bf16 parts, in order.  The weight gradient contracts over the blocks a, so its operands are the
 // columns of these arrays' 16-wide rows: the transposing LDS read (tr16_column8) forms them, with no second copy.
-// The weight gradient is fp32 exactly as the bands are (all kept products exact, fp32 sums).
+// The weight gradient is fp32 as the bands are (the same pairs of parts, fp32 sums).
 // Bound by issue: at K = 128 with silu 117 MFMAs and about 400 VALU instructions per wave and tile (gpre, its split)
 // fill 70% of the cycles at 3 waves per SIMD.  B=4 C=4096 L=8192 bf16: 478 us with silu, 201 identity (155 at K = 17:
 // 5.2 TB/s), against 1220 us for the three kernels.
@@ -251,6 +281,7 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
   constexpr int KP = F::KP, W = F::W, PX = F::PX, PG = F::PG;
   constexpr bool SILU = F::SILU;
   __shared__ __align__(16) unsigned char sm[F::BYTES];
+  static_assert((kConvTile + kConvMaxK) * 4 <= F::BYTES, "cconv_bwd_mma: a tile's gpre as fp32 in LDS");
   uint4* rev = reinterpret_cast<uint4*>(sm + F::O_REV);
   uint4* conv = reinterpret_cast<uint4*>(sm + F::O_CONV);
   uint16_t* xl = reinterpret_cast<uint16_t*>(sm + F::O_XL);
@@ -304,25 +335,28 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
     const int p0 = 16 * (32 * wave + li) + 4 * kk;  // the lane's positions in M-tile 2 wave; 256 on in the next
     q[0].load(gb, n0 + p0);
     q[1].load(gb, n0 + p0 + 256);
-    uint32_t b[2][4][PG];
+    uint32_t b[2][2][PG];  // pairs of positions
     if (n0 + 512 * wave < L) {
       nsq_bf16x8_t tap[S][kTapParts];
       get_band<S>(conv, tap);
       nsq_f32x4_t acc[2];
       band_run2<S, PX>(tap, xl, W, 32 * wave, 32 * wave + 16, acc[0], acc[1]);
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < 2; ++h) {
+        float gp[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float gp = n0 + p0 + 256 * h + r < L ? q[h].at(r) * dsilu(acc[h][r] + b0) : 0.f;
-          if (count) bacc += gp;
-          split_parts<PG>(gp, b[h][r]);
+          gp[r] = n0 + p0 + 256 * h + r < L ? q[h].at(r) * dsilu(acc[h][r] + b0) : 0.f;
+          if (count) bacc += gp[r];
         }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) split_parts2<PG>(gp[2 * r], gp[2 * r + 1], b[h][r]);
+      }
     } else {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < 2; ++r)
 #pragma unroll
           for (int p = 0; p < PG; ++p) b[h][r][p] = 0;
     }
@@ -330,8 +364,7 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
     for (int p = 0; p < PG; ++p)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        *reinterpret_cast<uint2*>(gl + p * W + p0 + 256 * h) =
-            make_uint2(b[h][0][p] | (b[h][1][p] << 16), b[h][2][p] | (b[h][3][p] << 16));
+        *reinterpret_cast<uint2*>(gl + p * W + p0 + 256 * h) = make_uint2(b[h][0][p], b[h][1][p]);
   };
   // gy itself into gl (identity)
   auto stage_g = [&]() {
@@ -369,6 +402,7 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
       __syncthreads();
     }
   }
+  bool bad = false;
   for (int g = g1 - 1; g >= g0; --g) {
     const int n0 = (g % ntiles) * kConvTile;
     if constexpr (SILU) carry(g % ntiles == ntiles - 1);
@@ -386,11 +420,14 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
       nsq_f32x4_t acc[2];
       band_run2<S, PG>(tap, gl, W, 32 * wave, 32 * wave + 16, acc[0], acc[1]);
       const RowBuf<DT, false> ob(gx + row_of(g), L);
+      float v[2][4];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const float v[4] = {acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
-        store4<DT, AL>(ob, n0 + 16 * (32 * wave + 16 * h + li) + 4 * kk, v);
-      }
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[h][r] = acc[h][r];
+      bad = bad || nonfinite(reinterpret_cast<const float(&)[8]>(v));
+#pragma unroll
+      for (int h = 0; h < 2; ++h) store4<DT, AL>(ob, n0 + 16 * (32 * wave + 16 * h + li) + 4 * kk, v[h]);
     }
     {
       // wave w contracts over blocks 32 w .. 32 w + 31
@@ -413,6 +450,43 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
     }
     __syncthreads();
   }
+#pragma unroll
+  for (int tg = 0; tg < F::TG; ++tg) {
+    const float v[4] = {D[tg][0], D[tg][1], D[tg][2], D[tg][3]};
+    bad = bad || nonfinite(v);
+  }
+  float wsum = 0.f;  // tap t's sum where it is taken directly
+  if (__syncthreads_or(bad || !(fabsf(bacc) < INFINITY))) {
+#pragma unroll
+    for (int tg = 0; tg < F::TG; ++tg) D[tg] = nsq_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    bacc = 0.f;
+    float* gp = reinterpret_cast<float*>(sm);  // gpre over [n0, n0 + kConvTile + K - 1)
+    const float* wc = w + int64_t(c) * K;
+#pragma unroll 1
+    for (int g = g0; g < g1; ++g) {
+      const int n0 = (g % ntiles) * kConvTile, count = min(kConvTile, L - n0);
+      const RowBuf<DT, false> xb(x + row_of(g), L), gb(gy + row_of(g), L), ob(gx + row_of(g), L);
+#pragma unroll 1
+      for (int m = t; m < kConvTile + K - 1; m += kConvThreads) {
+        float v = 0.f;
+        if (n0 + m < L) v = SILU ? gb.elem(n0 + m) * dsilu(direct_taps<DT>(xb, wc, K, n0 + m) + b0) : gb.elem(n0 + m);
+        gp[m] = v;
+        if (m < kConvTile) bacc += v;
+      }
+      __syncthreads();
+#pragma unroll 1
+      for (int m = t; m < count; m += kConvThreads) {
+        float a = 0.f;
+#pragma unroll 1
+        for (int j = 0; j < K; ++j) a = fmaf(wc[j], gp[m + K - 1 - j], a);
+        ob.store_elem(n0 + m, a);
+      }
+      if (t < K)
+#pragma unroll 1
+        for (int m = 0; m < count; ++m) wsum = fmaf(gp[m], xb.elem_halo(n0 + m - K + 1 + t), wsum);
+      __syncthreads();
+    }
+  }
   // fixed-order sums over the waves, then along the diagonals
   constexpr int RW = 16 * F::TG;
   float* red = reinterpret_cast<float*>(sm + F::O_REV);
@@ -432,7 +506,7 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
   if (t < K) {
     float s = 0.f;
     for (int i = 0; i < 16; ++i) s += red[i * RW + i + pad + t];
-    pw[t] = s;
+    pw[t] = s + wsum;
   }
 #pragma unroll
   for (int o = 32; o; o >>= 1) bacc += __shfl_xor(bacc, o);

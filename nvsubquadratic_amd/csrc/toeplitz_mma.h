@@ -28,14 +28,16 @@ template <int DT>
 constexpr int kParts = DT == NSQ_DTYPE_BF16 ? 1 : DT == NSQ_DTYPE_F16 ? 2 : 3;
 constexpr int kTapParts = 3;
 
-// v = sum of the parts, each a bf16 (its 16 bits), largest first.
+// (v0, v1) = sums of the parts, each a pair of bf16 in a word (v0 low), largest first.
 template <int P>
-__device__ __forceinline__ void split_parts(float v, uint32_t (&b)[P]) {
+__device__ __forceinline__ void split_parts2(float v0, float v1, uint32_t (&b)[P]) {
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const uint32_t u = __float_as_uint(v);
-    b[p] = u >> 16;
-    if (p + 1 < P) v -= __uint_as_float(u & 0xffff0000u);
+    b[p] = (__float_as_uint(v0) >> 16) | (__float_as_uint(v1) & 0xffff0000u);
+    if (p + 1 < P) {
+      v0 -= __uint_as_float(b[p] << 16);
+      v1 -= __uint_as_float(b[p] & 0xffff0000u);
+    }
   }
 }
 
@@ -50,6 +52,14 @@ __device__ __forceinline__ void mma_parts(const nsq_bf16x8_t (&tap)[kTapParts], 
 #pragma unroll
     for (int i = 0; i < P; ++i)
       if (d - i >= 0) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tap[d - i], x[i], c, 0, 0, 0);
+}
+
+// sum_j w[j] x[n - K + 1 + j], tap by tap from memory.
+template <int DT>
+__device__ __forceinline__ float direct_taps(const RowBuf<DT, false>& x, const float* __restrict__ w, int K, int n) {
+  float a = 0.f;
+  for (int j = 0; j < K; ++j) a = fmaf(w[j], x.elem_halo(n - K + 1 + j), a);
+  return a;
 }
 
 // The band of K taps as A operands.  conv: T[i][t] = w[t - i - pad] over the
@@ -81,11 +91,11 @@ __device__ __forceinline__ void band_operand(const float* wl, int K, int s, int 
   uint32_t u[kTapParts][4];
 #pragma unroll
   for (int e = 0; e < 8; e += 2) {
-    uint32_t a[kTapParts], b[kTapParts];
-    split_parts<kTapParts>(band_tap<S, REV>(wl, K, i, 32 * s + 8 * kk + e), a);
-    split_parts<kTapParts>(band_tap<S, REV>(wl, K, i, 32 * s + 8 * kk + e + 1), b);
+    uint32_t a[kTapParts];
+    split_parts2<kTapParts>(band_tap<S, REV>(wl, K, i, 32 * s + 8 * kk + e),
+                            band_tap<S, REV>(wl, K, i, 32 * s + 8 * kk + e + 1), a);
 #pragma unroll
-    for (int p = 0; p < kTapParts; ++p) u[p][e / 2] = a[p] | (b[p] << 16);
+    for (int p = 0; p < kTapParts; ++p) u[p][e / 2] = a[p];
   }
 #pragma unroll
   for (int p = 0; p < kTapParts; ++p) o[p] = make_uint4(u[p][0], u[p][1], u[p][2], u[p][3]);
@@ -137,11 +147,10 @@ struct PartChunk {
       uint32_t u[P][4];
 #pragma unroll
       for (int e = 0; e < 8; e += 2) {
-        uint32_t a[P], b[P];
-        split_parts<P>(w.at(e), a);
-        split_parts<P>(w.at(e + 1), b);
+        uint32_t a[P];
+        split_parts2<P>(w.at(e), w.at(e + 1), a);
 #pragma unroll
-        for (int p = 0; p < P; ++p) u[p][e / 2] = a[p] | (b[p] << 16);
+        for (int p = 0; p < P; ++p) u[p][e / 2] = a[p];
       }
 #pragma unroll
       for (int p = 0; p < P; ++p) o[p] = make_uint4(u[p][0], u[p][1], u[p][2], u[p][3]);

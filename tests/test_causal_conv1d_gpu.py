@@ -370,3 +370,100 @@ def test_bands_as_split_bf16_products(B, C, L, K, dtype, act):
         size = r.norm().item() if i < 2 else max(r.norm().item(), (r.numel() * B * L) ** 0.5)
         err = (a.double() - r).norm().item() / size
         assert err < (tol if i < 2 else 1e-6), (i, err)
+
+
+def _taps64(x, w, b, act):
+    """The conv tap by tap in float64: no zero tap meets a sample."""
+    K = w.shape[1]
+    xp = torch.nn.functional.pad(x, (K - 1, 0))
+    p = (xp.unfold(2, K, 1) * w[None, :, None, :]).sum(-1) + b.view(1, -1, 1)
+    return p * (1.0 / (1.0 + torch.exp(-p))) if act == "silu" else p
+
+
+def _same_kind(ref, got, skip=None):
+    """NaN where the reference has NaN, the same infinities, close elsewhere."""
+    ref, got = ref.double().cpu(), got.double().cpu()
+    keep = torch.ones_like(ref, dtype=torch.bool) if skip is None else ~skip
+    assert torch.equal(torch.isnan(ref)[keep], torch.isnan(got)[keep])
+    inf = torch.isinf(ref) & keep
+    assert torch.equal(ref[inf], got[inf])
+    fin = torch.isfinite(ref) & keep
+    assert torch.isfinite(got[fin]).all()
+    return fin
+
+
+@pytest.mark.parametrize("act", ["identity", "silu"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,C,L,K", [(1, 3, 400, 5), (2, 2, 4501, 9), (2, 2, 4504, 16), (1, 3, 2500, 17), (2, 3, 6200, 64),
+                                     (1, 2, 4300, 256), (1, 2048, 5 * 2048, 18)])
+def test_non_finite_samples_reach_their_own_outputs(B, C, L, K, dtype, act):
+    """An inf or NaN in x, in the upstream gradient or in a tap reaches the results that a sum over the taps gives, as
+    the same kind of value, and no other: not the outputs before it, nor the rest of its tile.  (Up to 16 taps the
+    register kernels pad the taps with zeros, which meet samples up to 16 before their own.)  Values elsewhere as
+    without it; 2048 channels: runs of tiles that start inside a row."""
+    print(f"B={B} C={C} L={L} K={K} {dtype} {act}", flush=True)
+    gen = torch.Generator().manual_seed(K)
+    x = torch.randn(B, C, L, generator=gen).to(dtype)
+    gy = torch.randn(B, C, L, generator=gen).to(dtype)
+    w, b = torch.randn(C, K, generator=gen) / K ** 0.5, torch.randn(C, generator=gen)
+    n = min(C, 3)  # channels checked
+    p1, p2 = L // 3, (2 * L) // 3
+    x[0, 0, p1], x[0, 0, p1 + 40], x[0, 1, p2] = float("inf"), float("-inf"), float("nan")
+    gy[0, 1, p1], gy[0, 0, p2] = float("-inf"), float("nan")
+    if C == 3:
+        w[2, K // 2] = float("inf")
+    xg, wg, bg = (t.cuda().requires_grad_() for t in (x, w, b))
+    y = causal_conv1d(xg, wg, bg, act)
+    gx, gw, gb = torch.autograd.grad(y, (xg, wg, bg), gy.cuda())
+
+    x6, w6, b6 = (t[:, :n].double() if t.dim() == 3 else t[:n].double() for t in (x, w, b))
+    p = _taps64(x6, w6, b6, "identity")
+    s = 1.0 / (1.0 + torch.exp(-p))
+    g6 = gy[:, :n].double()
+    gp = g6 * (s * (1.0 + p * (1.0 - s))) if act == "silu" else g6
+    want_gx = (torch.nn.functional.pad(gp, (0, K - 1)).unfold(2, K, 1) * w6.flip(1)[None, :, None, :]).sum(-1)
+    xw = torch.nn.functional.pad(x6, (K - 1, 0)).unfold(2, K, 1)  # [B, n, L, K]
+    want_gw, want_gb = (gp.unsqueeze(-1) * xw).sum((0, 2)), gp.sum((0, 2))
+    want_y = p * s if act == "silu" else p
+    pad = 16 - K if K <= 16 else 0
+
+    def near(bad):  # positions within `pad` of a non-finite result
+        m = torch.zeros_like(bad)
+        for i in range(1, pad + 1):
+            m |= torch.roll(bad, i, -1) | torch.roll(bad, -i, -1)
+        return m & ~bad
+
+    tol = {torch.float32: 2e-5, torch.bfloat16: 2e-2, torch.float16: 4e-3}[dtype]
+    for want, got in ((want_y, y[:, :n]), (want_gx, gx[:, :n])):
+        fin = _same_kind(want, got, near(~torch.isfinite(want)) if pad else None)
+        a, r = got.double().cpu()[fin], want[fin]
+        assert (a - r).norm() < tol * r.norm()
+    if not pad:
+        for want, got in ((want_gw, gw[:n]), (want_gb, gb[:n])):
+            _same_kind(want, got)
+
+
+@pytest.mark.parametrize("K", [9, 64, 256])
+def test_values_above_the_largest_bf16_stay_finite(K):
+    """fp32 values between the largest bf16 and the largest fp32 (which round to infinity in bf16) as samples, taps and
+    gradients: results as in float64."""
+    B, C, L = 1, 2, 3000
+    gen = torch.Generator().manual_seed(K)
+    x, gy = torch.randn(B, C, L, generator=gen), torch.randn(B, C, L, generator=gen)
+    w, b = torch.randn(C, K, generator=gen) * 1e-3, torch.randn(C, generator=gen)
+    big = float(torch.finfo(torch.float32).max)
+    x[0, 0, 700], gy[0, 0, 1500], w[1, 3] = big, -big, big
+    x[0, 1] *= 1e-3
+    gy[0, 1] *= 1e-3
+    args = [t.cuda().requires_grad_() for t in (x, w, b)]
+    y = causal_conv1d(*args)
+    got = (y, *torch.autograd.grad(y, args, gy.cuda()))
+    args6 = [t.double().requires_grad_() for t in (x, w, b)]
+    y6 = _taps64(*args6, "identity")
+    want = (y6, *torch.autograd.grad(y6, args6, gy.double()))
+    for i, (a, r) in enumerate(zip(got, want)):
+        for c in range(C):  # the channels differ in size by 1e38
+            ac, rc = (t[:, c] if t.dim() == 3 else t[c] for t in (a.double().cpu(), r))
+            if rc.abs().max() < 1e38:  # an overflowing sum is an infinity in any order
+                assert torch.isfinite(ac).all(), (i, c)
+                assert (ac - rc).norm() <= 1e-5 * rc.norm(), (i, c)
