@@ -5,12 +5,17 @@
 //     Y = T Xw,   T[i][t] = band[t - i],   Xw[t][a] = src[16 a + t],
 // t < 32 S.  The bf16 matrix rate is 16 times the fp32 one, so every fp32
 // operand is written as a sum of bf16 values and the product runs once per
-// pair of parts.  Parts are cut off, not rounded, so the sum is the operand
-// exactly and no part overflows:
+// pair of parts.  Each part is what the parts before it leave, rounded to
+// nearest; the sum is the operand exactly:
 //     fp32: 3 parts (8 + 8 + 8 mantissa bits), fp16: 2 (8 + 3), bf16: 1.
-// The pairs (i, j) with i + j <= 2 are kept: the dropped ones are below 2^-24
-// of the largest, the rounding of an fp32 product.  bf16 samples against fp32
-// taps are 3 products (none dropped), i.e. 3/16 of the fp32 matrix time.
+// The pairs (i, j) with i + j <= 2 are kept.  For an operand in [1, 2) part 1
+// is at most 2^-8 and part 2 at most 2^-17, so the dropped pairs, (1, 2) and
+// (2, 1) above all, are at most 2^-24 of the product: what one fp32 rounding
+// may lose, and of either sign.  (Parts cut off instead of rounded reach 2^-7
+// and 2^-15 with the operand's sign: 2^-21, always towards zero.)  bf16
+// samples against fp32 taps are 3 products (none dropped), i.e. 3/16 of the
+// fp32 matrix time.  Operands below 2^-110 lose parts to bf16's smallest
+// value.
 //
 // Lane layout: lane l supplies A[l % 16][8 (l / 16) + e] and B[8 (l / 16) +
 // e][l % 16], e < 8, and receives D[4 (l / 16) + r][l % 16].  With the taps as
@@ -33,7 +38,7 @@ template <int P>
 __device__ __forceinline__ void split_parts2(float v0, float v1, uint32_t (&b)[P]) {
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    b[p] = (__float_as_uint(v0) >> 16) | (__float_as_uint(v1) & 0xffff0000u);
+    b[p] = f32x2_to_bf16x2_bits(v0, v1);
     if (p + 1 < P) {
       v0 -= __uint_as_float(b[p] << 16);
       v1 -= __uint_as_float(b[p] & 0xffff0000u);
