@@ -189,9 +189,9 @@ cconv_fwd_mma_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __
   PartChunk<DT, AL> cm, cx;  // samples [8t, 8t + 8) of the window and, for the first threads, [2048 + 8t, ...)
   auto load = [&](int g) {
     const int b = g / ntiles, n0 = (g - b * ntiles) * kConvTile;
-    const RowBuf<DT, false> rb(x + (int64_t(b) * C + c) * L, L);
-    cm.load(rb, n0 - KP + 8 * t);
-    if (t < KP / 8) cx.load(rb, n0 - KP + kConvTile + 8 * t);
+    const typename Elem<DT>::T* row = x + (int64_t(b) * C + c) * L;
+    cm.load(row, n0 - KP + 8 * t, L);
+    if (t < KP / 8) cx.load(row, n0 - KP + kConvTile + 8 * t, L);
   };
   load(g0);
   __syncthreads();  // taps staged
@@ -220,7 +220,6 @@ cconv_fwd_mma_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __
     if (n0 + 512 * wave >= L) continue;
     nsq_f32x4_t acc[2];
     band_run2<S, P>(tap, xb, W, 32 * wave, 32 * wave + 16, acc[0], acc[1]);
-    const RowBuf<DT, false> ob(y + (int64_t(b) * C + c) * L, L);
     float v[2][4];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -231,7 +230,7 @@ cconv_fwd_mma_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[h][r] = act_fwd<ACT>(v[h][r]);
-      store4<DT, AL>(ob, n0 + p0 + 256 * h, v[h]);
+      store4<DT, AL>(y + (int64_t(b) * C + c) * L, n0 + p0 + 256 * h, L, v[h]);
     }
   }
 #pragma unroll 1
@@ -301,13 +300,11 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
   auto row_of = [&](int g) { return (int64_t(g / ntiles) * C + c) * L; };
   auto load = [&](int g) {
     const int n0 = (g % ntiles) * kConvTile;
-    const RowBuf<DT, false> rb(x + row_of(g), L);
-    xm.load(rb, n0 - KP + 8 * t);
-    if (t < KP / 8) xx.load(rb, n0 - KP + kConvTile + 8 * t);
+    xm.load(x + row_of(g), n0 - KP + 8 * t, L);
+    if (t < KP / 8) xx.load(x + row_of(g), n0 - KP + kConvTile + 8 * t, L);
     if constexpr (!SILU) {
-      const RowBuf<DT, false> gb(gy + row_of(g), L);
-      gm.load(gb, n0 + 8 * t);
-      if (t < KP / 8) gx8.load(gb, n0 + kConvTile + 8 * t);
+      gm.load(gy + row_of(g), n0 + 8 * t, L);
+      if (t < KP / 8) gx8.load(gy + row_of(g), n0 + kConvTile + 8 * t, L);
     }
   };
   load(g1 - 1);
@@ -330,11 +327,10 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
   // gpre of tile g into gl (SILU)
   auto make_gpre = [&](int g, bool count) {
     const int n0 = (g % ntiles) * kConvTile;
-    const RowBuf<DT, false> gb(gy + row_of(g), L);
     Quad<DT, AL> q[2];
     const int p0 = 16 * (32 * wave + li) + 4 * kk;  // the lane's positions in M-tile 2 wave; 256 on in the next
-    q[0].load(gb, n0 + p0);
-    q[1].load(gb, n0 + p0 + 256);
+    q[0].load(gy + row_of(g), n0 + p0, L);
+    q[1].load(gy + row_of(g), n0 + p0 + 256, L);
     uint32_t b[2][2][PG];  // pairs of positions
     if (n0 + 512 * wave < L) {
       nsq_bf16x8_t tap[S][kTapParts];
@@ -419,7 +415,6 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
       get_band<S>(rev, tap);
       nsq_f32x4_t acc[2];
       band_run2<S, PG>(tap, gl, W, 32 * wave, 32 * wave + 16, acc[0], acc[1]);
-      const RowBuf<DT, false> ob(gx + row_of(g), L);
       float v[2][4];
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -427,7 +422,7 @@ __attribute__((amdgpu_waves_per_eu(CconvBwdCfg<DT, S, ACT>::BYTES > 80 * 1024 ? 
         for (int r = 0; r < 4; ++r) v[h][r] = acc[h][r];
       bad = bad || nonfinite(reinterpret_cast<const float(&)[8]>(v));
 #pragma unroll
-      for (int h = 0; h < 2; ++h) store4<DT, AL>(ob, n0 + 16 * (32 * wave + 16 * h + li) + 4 * kk, v[h]);
+      for (int h = 0; h < 2; ++h) store4<DT, AL>(gx + row_of(g), n0 + 16 * (32 * wave + 16 * h + li) + 4 * kk, L, v[h]);
     }
     {
       // wave w contracts over blocks 32 w .. 32 w + 31

@@ -136,18 +136,56 @@ __device__ __forceinline__ void get_band(const uint4* from, nsq_bf16x8_t (&tap)[
     }
 }
 
+// Rows that are not whole 16-byte chunks (AL false) are read and written as unaligned vectors, and by elements only
+// where a chunk crosses the row's end.  Element accesses alone (a lane's eight at a stride of 16 or 32 bytes across
+// lanes) took B=4 C=512 L=10007 K=33 from 27 (row-wise loads of the fp32 products) to 51 us forward in bf16.
+template <int DT, int N>
+struct RowVec {  // N elements of DT as a vector that may start at any element
+  static constexpr int W = N * int(sizeof(typename Elem<DT>::T)) / 4;
+  typedef uint32_t V __attribute__((ext_vector_type(W), aligned(sizeof(typename Elem<DT>::T))));
+};
+
+// row[n, n + N) as words, zero outside [0, L); a chunk before the row lies wholly before it.
+template <int DT, int N, int W>
+__device__ __forceinline__ void load_any(const typename Elem<DT>::T* __restrict__ row, const RowBuf<DT, false>& rb,
+                                         int n, int L, uint32_t (&w)[W]) {
+  using R = RowVec<DT, N>;
+  static_assert(W == R::W, "load_any: words");
+  uint32_t v[W];
+#pragma unroll
+  for (int i = 0; i < W; ++i) v[i] = 0;
+  if (n >= 0 && n + N <= L) {
+    const typename R::V m = *reinterpret_cast<const typename R::V*>(row + n);
+#pragma unroll
+    for (int i = 0; i < W; ++i) v[i] = m[i];
+  } else if (n >= 0 && n < L) {
+    if constexpr (DT == NSQ_DTYPE_F32) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = rb.elem_halo_bits(n + i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < W; ++i) v[i] = rb.elem_halo_bits(n + 2 * i) | (rb.elem_halo_bits(n + 2 * i + 1) << 16);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < W; ++i) w[i] = v[i];
+}
+
 // Eight consecutive samples of a row, loaded raw and written out as bf16 parts.
 template <int DT, bool AL>
 struct PartChunk {
   static constexpr int P = kParts<DT>;
-  Win8<DT, AL> w;
-  __device__ __forceinline__ void load(const RowBuf<DT, false>& rb, int n) { w.load(rb, n); }
+  Win8<DT, true> w;
+  __device__ __forceinline__ void load(const typename Elem<DT>::T* __restrict__ row, int n, int L) {
+    const RowBuf<DT, false> rb(row, L);
+    if constexpr (AL)
+      w.load(rb, n);
+    else
+      load_any<DT, 8>(row, rb, n, L, w.w);
+  }
   __device__ __forceinline__ void parts(uint4 (&o)[P]) const {
-    if constexpr (DT == NSQ_DTYPE_BF16 && AL) {
+    if constexpr (DT == NSQ_DTYPE_BF16) {
       o[0] = make_uint4(w.w[0], w.w[1], w.w[2], w.w[3]);
-    } else if constexpr (DT == NSQ_DTYPE_BF16) {
-      o[0] = make_uint4(w.w[0] | (w.w[1] << 16), w.w[2] | (w.w[3] << 16), w.w[4] | (w.w[5] << 16),
-                        w.w[6] | (w.w[7] << 16));
     } else {
       uint32_t u[P][4];
 #pragma unroll
@@ -163,27 +201,37 @@ struct PartChunk {
   }
 };
 
-// Four consecutive outputs at position n of a row (n a multiple of 4): one 8- or 16-byte store where the rows allow
-// (AL: the row length a multiple of 8 / 4 elements, 16-byte aligned), element stores dropped past the end otherwise.
+// Four consecutive outputs at position n of a row (n a multiple of 4), dropped past the end: one 8- or 16-byte store,
+// aligned where the rows are (AL), else by elements where it crosses the end.
 template <int DT, bool AL>
-__device__ __forceinline__ void store4(const RowBuf<DT, false>& rb, int n, const float (&v)[4]) {
+__device__ __forceinline__ void store4(typename Elem<DT>::T* __restrict__ row, int n, int L, const float (&v)[4]) {
+  const RowBuf<DT, false> rb(row, L);
+  using R = RowVec<DT, 4>;
+  uint32_t u[R::W];
+  if constexpr (DT == NSQ_DTYPE_F32) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = __float_as_uint(v[i]);
+  } else if constexpr (DT == NSQ_DTYPE_BF16) {
+    u[0] = f32x2_to_bf16x2_bits(v[0], v[1]);
+    u[1] = f32x2_to_bf16x2_bits(v[2], v[3]);
+  } else {
+    u[0] = __builtin_bit_cast(uint32_t, __floats2half2_rn(v[0], v[1]));
+    u[1] = __builtin_bit_cast(uint32_t, __floats2half2_rn(v[2], v[3]));
+  }
   if constexpr (AL) {
     using U2 = uint32_t __attribute__((ext_vector_type(2)));
     using U4 = uint32_t __attribute__((ext_vector_type(4)));
     const int off = n * int(sizeof(typename Elem<DT>::T));
-    if constexpr (DT == NSQ_DTYPE_F32) {
-      __builtin_amdgcn_raw_buffer_store_b128(
-          U4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, rb.r, off, 0,
-          0);
-    } else if constexpr (DT == NSQ_DTYPE_BF16) {
-      __builtin_amdgcn_raw_buffer_store_b64(U2{f32x2_to_bf16x2_bits(v[0], v[1]), f32x2_to_bf16x2_bits(v[2], v[3])},
-                                            rb.r, off, 0, 0);
-    } else {
-      __builtin_amdgcn_raw_buffer_store_b64(U2{__builtin_bit_cast(uint32_t, __floats2half2_rn(v[0], v[1])),
-                                               __builtin_bit_cast(uint32_t, __floats2half2_rn(v[2], v[3]))},
-                                            rb.r, off, 0, 0);
-    }
-  } else {
+    if constexpr (DT == NSQ_DTYPE_F32)
+      __builtin_amdgcn_raw_buffer_store_b128(U4{u[0], u[1], u[2], u[3]}, rb.r, off, 0, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b64(U2{u[0], u[1]}, rb.r, off, 0, 0);
+  } else if (n + 4 <= L) {
+    typename R::V m;
+#pragma unroll
+    for (int i = 0; i < R::W; ++i) m[i] = u[i];
+    *reinterpret_cast<typename R::V*>(row + n) = m;
+  } else if (n < L) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) rb.store_elem(n + r, v[r]);
   }
@@ -193,24 +241,22 @@ __device__ __forceinline__ void store4(const RowBuf<DT, false>& rb, int n, const
 template <int DT, bool AL>
 struct Quad {
   static constexpr bool HALF = DT != NSQ_DTYPE_F32;
-  static constexpr int W = (HALF && AL) ? 2 : 4;
-  uint32_t w[W];
-  __device__ __forceinline__ void load(const RowBuf<DT, false>& rb, int n) {
-    const int off = n * int(sizeof(typename Elem<DT>::T));
-    if constexpr (AL && HALF) {
-      const auto m = __builtin_amdgcn_raw_buffer_load_b64(rb.r, off, 0, 0);
+  uint32_t w[HALF ? 2 : 4];
+  __device__ __forceinline__ void load(const typename Elem<DT>::T* __restrict__ row, int n, int L) {
+    const RowBuf<DT, false> rb(row, L);
+    if constexpr (!AL) {
+      load_any<DT, 4>(row, rb, n, L, w);
+    } else if constexpr (HALF) {
+      const auto m = __builtin_amdgcn_raw_buffer_load_b64(rb.r, n * 2, 0, 0);
       w[0] = m[0]; w[1] = m[1];
-    } else if constexpr (AL) {
-      const auto m = __builtin_amdgcn_raw_buffer_load_b128(rb.r, off, 0, 0);
+    } else {
+      const auto m = __builtin_amdgcn_raw_buffer_load_b128(rb.r, n * 4, 0, 0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) w[i] = m[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = rb.elem_halo_bits(n + i);
     }
   }
   __device__ __forceinline__ float at(int i) const {
-    if constexpr (HALF && AL) {
+    if constexpr (HALF) {
       const uint32_t v = (i & 1) ? (w[i >> 1] >> 16) : (w[i >> 1] & 0xffffu);
       return RowBuf<DT, false>::bits_to_f32(v);
     } else {

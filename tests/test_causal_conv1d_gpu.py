@@ -498,3 +498,35 @@ def test_split_products_round_to_nearest(dtype):
     assert err.abs().max() <= 3 * 2.0 ** -24
     if dtype == torch.float32:
         assert err.mean().abs() <= 2.0 ** -25
+
+
+@pytest.mark.parametrize("act", ["identity", "silu"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("L", [3, 8, 2045, 2047, 2048, 2049, 2052, 4100])
+def test_unaligned_rows(L, dtype, act):
+    """Rows that start at any element and end inside a vector of 4 or 8: odd lengths, and tensors one to three elements
+    into their storage, against the same values in aligned storage where that exists, else float64.  What lies beside
+    the tensor in its storage is NaN: nothing outside a row is read, and nothing is written there."""
+    gen = torch.Generator().manual_seed(L)
+    B, C, K = 2, 3, 17
+    nan = float("nan")
+
+    def at(t, off):  # a contiguous copy of t, `off` elements into a NaN-filled storage
+        flat = torch.full((t.numel() + 16,), nan, device="cuda", dtype=t.dtype)
+        v = flat[off:off + t.numel()].view(t.shape)
+        v.copy_(t)
+        return v
+
+    x, gy = (torch.randn(B, C, L, generator=gen).to(dtype) for _ in range(2))
+    w, b = torch.randn(C, K, generator=gen) / K ** 0.5, torch.randn(C, generator=gen)
+    x6, w6, b6 = (t.double().requires_grad_() for t in (x, w, b))
+    y6 = _taps64(x6, w6, b6, act)
+    want = (y6, *torch.autograd.grad(y6, (x6, w6, b6), gy.double()))
+    tol = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]
+    for off in range(4):
+        args = [at(x, off).requires_grad_(), w.cuda().requires_grad_(), b.cuda().requires_grad_()]
+        y = causal_conv1d(*args, act)
+        got = (y, *torch.autograd.grad(y, args, at(gy, (off + 1) % 4)))
+        for i, (r, a) in enumerate(zip(want, got)):
+            err = (a.double().cpu() - r).norm() / r.norm()
+            assert err < (tol if i < 2 else 2e-6), (off, i, float(err))
