@@ -68,24 +68,32 @@ static bool rows16(int64_t L, const void* a, const void* b, const void* c) {
 
 constexpr int kConvSegTiles = 4;  // tiles per workgroup of the register backward
 // The register kernels run up to 4 taps, the matrix-core ones above 16; between, by what measured faster (us, register /
-// matrix-core).  B=4 C=4096 L=8192 (2^27 samples):
+// matrix-core).  Large calls, B=4 C=4096 L=8192 (2^27 samples):
 //   forward, bf16:  identity K = 8 93 / 101, K = 9 112 / 101;  silu K = 4 117 / 105, K = 5 135 / 105;
 //   forward, fp32:  K = 4 198 / 201, K = 5 218 / 201, K = 16 226 / 201 (either activation);
 //   backward, bf16: silu K = 4 196 / 218, K = 5 274 / 218;  fp32: silu K = 4 339 / 317, K = 5 417 / 317.
-// Below 2^25 samples with aligned rows the matrix-core kernels' setup (bands, staging) shows, in fp32 up to 16 taps
-// forward (B=4 C=1024 L=2048, silu: K = 16 13.2 / 14.3) and 8 backward (K = 7 25.6 / 27.2), in 16 bits up to 8 forward
-// (K = 7 9.4 / 11.1); unaligned rows favour them from 5 taps (B=8 C=768 L=777 fp32, K = 7 25.8 / 18.0).
+// With fewer samples the matrix-core kernels' setup (bands, staging, the tile beside a run's) shows.  Aligned rows, forward:
+//   fp32 up to 16 taps and 16 bits up to 8 to 2^25 (there fp32 39.5 / 42.0, fp16 33.3 / 35.3, bf16 35.4 / 31.5; B=4 C=1024 L=2048, silu: fp32 K = 16 13.2 / 14.3, bf16 K = 7
+//   9.4 / 11.1); 16 bits up to 16 taps while launches dominate, to 2^19 samples in bf16 (2.4 / 2.6, at 2^20 3.1 / 2.9) and
+//   2^23 in fp16, whose samples are two parts (2^22 5.7 / 5.9).
+// Aligned rows, forward + backward, up to 8 taps: fp32 below 2^25 (K = 7 25.6 / 27.2 backward), bf16 to 2^23 (B=2 C=512
+//   L=8192 silu K = 5 36.8 / 41.8; at 2^24 62 / 62), fp16 to 2^24 (63 / 71).
+// Unaligned rows: the matrix-core kernels read and write them as vectors (toeplitz_mma.h), so they take all calls from 5
+// taps but the 16-bit identity forward up to 8 (B=8 C=768 L=777 fp32, K = 7 25.8 / 18.0).
 constexpr int kConvShortMax = 4;
 constexpr int64_t kConvSmall = int64_t(1) << 25;
 template <int DT>
 static bool short_fwd(int K, int act, int64_t samples, bool aligned) {
-  constexpr bool F32 = DT == NSQ_DTYPE_F32;
-  return K <= kConvShortMax || (K <= 8 && act == NSQ_ACT_IDENTITY && !F32) ||
-         (K <= (F32 ? 16 : 8) && aligned && samples < kConvSmall);
+  if (K <= kConvShortMax || (K <= 8 && act == NSQ_ACT_IDENTITY && DT != NSQ_DTYPE_F32)) return true;
+  if (!aligned || K > 16) return false;
+  const int64_t few = DT == NSQ_DTYPE_F32 ? kConvSmall : int64_t(1) << (DT == NSQ_DTYPE_BF16 ? 19 : 23);
+  return samples <= few || (K <= 8 && samples <= kConvSmall - (DT == NSQ_DTYPE_BF16));
 }
 template <int DT>
 static bool short_bwd(int K, int64_t samples, bool aligned) {
-  return K <= kConvShortMax || (DT == NSQ_DTYPE_F32 && K <= 8 && aligned && samples < kConvSmall);
+  if (K <= kConvShortMax) return true;
+  const int64_t few = DT == NSQ_DTYPE_F32 ? kConvSmall - 1 : int64_t(1) << (DT == NSQ_DTYPE_BF16 ? 23 : 24);
+  return K <= 8 && aligned && samples <= few;
 }
 
 __global__ void cconv_wgrad_reduce_kernel(const float* __restrict__ part, int nparts, int K, float* __restrict__ gw,
@@ -111,7 +119,11 @@ static int64_t cconv_wgrad_parts(int64_t B, int64_t L) {
 // owns one channel and walks a run of its (batch row, 2048-output tile)
 // sequence, so the split taps are prepared once per run.
 // ---------------------------------------------------------------------------
-constexpr int kMmaTarget = 4096;  // workgroups wanted: 4 or more per resident slot (256 CUs x 2..4)
+// Workgroups wanted: 4 or more per resident slot (256 CUs x 2..4) so that they end together, but one where tiles are
+// few: a run pays for its bands, and with silu for the gpre of the tile beside it, which is half of a run of one.
+// Measured, 1024 / 4096 (us, forward + backward): B=2 C=128 L=16384 K=33 bf16 (2048 tiles) 21.4 / 27.8; 8192 tiles
+// 6% better, 32768 1.5% worse on average and up to 9%.
+inline int64_t mma_target(int64_t tiles) { return tiles <= 8192 ? 1024 : 4096; }
 
 // A band multiplies every sample of a block's window, later ones too, by some zero tap, and inf leaves NaN among its
 // parts (inf - inf; a finite value above the largest bf16 is inf in its first part): a non-finite value makes all the
@@ -126,9 +138,9 @@ __device__ __forceinline__ bool nonfinite(const float (&v)[N]) {
   return !(s[0] + s[1] == 0.f);
 }
 
-// Tiles per run: as many as leave kMmaTarget workgroups, at least 1.
+// Tiles per run: as many as leave mma_target workgroups, at least 1.
 static int64_t mma_run_tiles(int64_t B, int64_t C, int64_t L) {
-  const int64_t tiles = B * ceil_div(L, kConvTile), want = ceil_div(kMmaTarget, C);
+  const int64_t tiles = B * ceil_div(L, kConvTile), want = ceil_div(mma_target(C * tiles), C);
   return tiles / want > 1 ? tiles / want : 1;
 }
 static int64_t mma_runs(int64_t B, int64_t C, int64_t L) {
@@ -675,7 +687,7 @@ static void launch_bwd_short(const void* gy, const void* x, const float* w, cons
     if (K <= 4)
       hipLaunchKernelGGL((cconv_bwd_short_kernel<DT, A, F, 4>), grid, dim3(kConvThreads), 0, st, (const ET*)gy,
                          (const ET*)x, w, bias, (ET*)gx, ws, B, C, L, K);
-    else if constexpr (A && DT == NSQ_DTYPE_F32)
+    else if constexpr (A)
       hipLaunchKernelGGL((cconv_bwd_short_kernel<DT, A, F, 8>), grid, dim3(kConvThreads), 0, st, (const ET*)gy,
                          (const ET*)x, w, bias, (ET*)gx, ws, B, C, L, K);
   };
@@ -708,7 +720,7 @@ static void launch_fwd(const void* x, const float* w, const float* bias, void* y
       if (K <= 8)
         hipLaunchKernelGGL((cconv_fwd_short_kernel<DT, A, F, 8>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
                            bias, (ET*)y, C, L, K);
-      else if constexpr (A && DT == NSQ_DTYPE_F32)
+      else if constexpr (A)
         hipLaunchKernelGGL((cconv_fwd_short_kernel<DT, A, F, 16>), grid, dim3(kConvThreads), 0, st, (const ET*)x, w,
                            bias, (ET*)y, C, L, K);
     }
@@ -773,7 +785,7 @@ static float* noalloc_scratch() {
 
 // What the noalloc entry point counts against its scratch, which fixes the shapes it takes: partials of one run per
 // kConvSegTiles tiles, and for silu above 16 taps an fp32 row set [B, C, L].  Never less than the backward
-// uses where that fits (at most max(C, kMmaTarget + C) partial rows).
+// uses where that fits (at most max(C, 4096 + C) partial rows).
 static size_t noalloc_bytes(int64_t B, int64_t C, int64_t L, int64_t K, int act) {
   const int64_t pre = act == NSQ_ACT_SILU && K > 16 ? B * C * L : 0;
   const size_t was = size_t(pre + C * cconv_wgrad_parts(B, L) * (K + 1)) * sizeof(float);
