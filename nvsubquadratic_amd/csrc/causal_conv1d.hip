@@ -72,10 +72,11 @@ constexpr int kConvSegTiles = 4;  // tiles per workgroup of the register backwar
 //   forward, bf16:  identity K = 8 93 / 101, K = 9 112 / 101;  silu K = 4 117 / 105, K = 5 135 / 105;
 //   forward, fp32:  K = 4 198 / 201, K = 5 218 / 201, K = 16 226 / 201 (either activation);
 //   backward, bf16: silu K = 4 196 / 218, K = 5 274 / 218;  fp32: silu K = 4 339 / 317, K = 5 417 / 317.
-// With fewer samples the matrix-core kernels' setup (bands, staging, the tile beside a run's) shows.  Aligned rows, forward:
-//   fp32 up to 16 taps and 16 bits up to 8 to 2^25 (there fp32 39.5 / 42.0, fp16 33.3 / 35.3, bf16 35.4 / 31.5; B=4 C=1024 L=2048, silu: fp32 K = 16 13.2 / 14.3, bf16 K = 7
-//   9.4 / 11.1); 16 bits up to 16 taps while launches dominate, to 2^19 samples in bf16 (2.4 / 2.6, at 2^20 3.1 / 2.9) and
-//   2^23 in fp16, whose samples are two parts (2^22 5.7 / 5.9).
+// With fewer samples the matrix-core kernels' setup (bands, staging, the tile beside a run's) shows.  Aligned rows,
+// forward: fp32 up to 16 taps and 16 bits up to 8 to 2^25 (there fp32 39.5 / 42.0, fp16 33.3 / 35.3, but bf16 35.4 /
+//   31.5; B=4 C=1024 L=2048, silu: fp32 K = 16 13.2 / 14.3, bf16 K = 7 9.4 / 11.1); 16 bits up to 16 taps while
+//   launches dominate, to 2^19 samples in bf16 (2.4 / 2.6, at 2^20 3.1 / 2.9) and 2^23 in fp16, whose samples are two
+//   parts (2^22 5.7 / 5.9).
 // Aligned rows, forward + backward, up to 8 taps: fp32 below 2^25 (K = 7 25.6 / 27.2 backward), bf16 to 2^23 (B=2 C=512
 //   L=8192 silu K = 5 36.8 / 41.8; at 2^24 62 / 62), fp16 to 2^24 (63 / 71).
 // Unaligned rows: the matrix-core kernels read and write them as vectors (toeplitz_mma.h), so they take all calls from 5
@@ -121,8 +122,8 @@ static int64_t cconv_wgrad_parts(int64_t B, int64_t L) {
 // ---------------------------------------------------------------------------
 // Workgroups wanted: 4 or more per resident slot (256 CUs x 2..4) so that they end together, but one where tiles are
 // few: a run pays for its bands, and with silu for the gpre of the tile beside it, which is half of a run of one.
-// Measured, 1024 / 4096 (us, forward + backward): B=2 C=128 L=16384 K=33 bf16 (2048 tiles) 21.4 / 27.8; 8192 tiles
-// 6% better, 32768 1.5% worse on average and up to 9%.
+// Measured, 1024 / 4096 (us, forward + backward): B=2 C=128 L=16384 K=33 bf16 (2048 tiles) silu 27.0 / 32.5, identity
+// 16.7 / 19.7; 8192 tiles 6% better on average, 32768 1.5% worse and up to 9%.
 inline int64_t mma_target(int64_t tiles) { return tiles <= 8192 ? 1024 : 4096; }
 
 // A band multiplies every sample of a block's window, later ones too, by some zero tap, and inf leaves NaN among its
