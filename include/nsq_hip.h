@@ -39,7 +39,8 @@ enum {
 
 enum { NSQ_DTYPE_F32 = 0, NSQ_DTYPE_BF16 = 1, NSQ_DTYPE_F16 = 2 };
 
-enum { NSQ_DIR_FWD = 0, NSQ_DIR_BWD = 1 };
+/* NSQ_DIR_STATE (2D / 3D convolutions): the bytes a forward may leave for its backward. */
+enum { NSQ_DIR_FWD = 0, NSQ_DIR_BWD = 1, NSQ_DIR_STATE = 2 };
 
 /* Library version of this ABI (NSQ_ABI_VERSION). */
 int nsq_abi_version(void);
@@ -254,8 +255,11 @@ int nsq_causal_conv1d_bwd(const void* gy, const void* x, const float* weight, co
  * workspace.  It has no counterpart in the reference: it is for callers that
  * cannot allocate device memory, such as code under HIP graph capture or a
  * serving loop that forbids allocation.  It calls no hipMalloc / hipFree.
- * Shapes whose scratch (nsq_causal_conv1d_bwd_workspace_bytes) exceeds the
- * buffer return NSQ_ERR_UNSUPPORTED without launching anything.  Every call
+ * It takes the shapes it always took: those for which the weight-gradient
+ * partials (nsq_causal_conv1d_bwd_workspace_bytes) and, with silu above 16
+ * taps, an fp32 array [B, C, L] (which the kernels no longer need) fit the
+ * buffer together.  The others return NSQ_ERR_UNSUPPORTED without launching
+ * anything; some of them would fit a workspace of that size.  Every call
  * on one GPU shares that GPU's buffer: calls that overlap on one GPU (other
  * streams, other threads) race and must be serialised by the caller.
  */
@@ -305,7 +309,9 @@ size_t nsq_fftconv_nd_workspace_bytes(int nd, int64_t B, int64_t H, const int64_
                                       int64_t kbatch, int direction);
 /* A forward given a workspace of the backward's size keeps the transformed x
  * and the filter spectrum in it; a backward called on that untouched workspace
- * with fwd_state = 1 reuses them (results identical to fwd_state = 0). */
+ * with fwd_state = 1 reuses them (results identical to fwd_state = 0).  Shapes
+ * whose forward keeps nothing (small 2D planes) ignore fwd_state; for them the
+ * query with NSQ_DIR_STATE is 0, for the others it is the backward's size. */
 
 int nsq_fftconv_nd_fwd(int nd, const void* x, const float* k, const void* shortcut, void* y, int dtype, int64_t B,
                        int64_t H, const int64_t* S, const int64_t* K, int64_t kbatch, void* workspace,

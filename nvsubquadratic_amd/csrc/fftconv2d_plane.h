@@ -344,7 +344,8 @@ __global__ __launch_bounds__(P::T) void plane2_fwd_kernel(const typename Elem<DT
   float2* lds = reinterpret_cast<float2*>(plane2_sm);
   const Plane2Io<DT, P, GATED> io(g, plane2_sm);
   const Plane2Roots<P> tw(lds + P::F0 * P::RS, roots);
-  const int h = int(blockIdx.x), b0 = int(blockIdx.y) * g.per_wg, b1 = min(g.B, b0 + g.per_wg);
+  const int share = int(blockIdx.x / unsigned(g.H)), h = int(blockIdx.x) - share * g.H;
+  const int b0 = share * g.per_wg, b1 = min(g.B, b0 + g.per_wg);
   const int64_t hk = g.kfilm ? int64_t(b0) * g.H + h : h;
   Plane2Vec<DT> xv[4], kg[4];
   io.load(x, b0, h, xv);
@@ -403,8 +404,8 @@ __global__ __launch_bounds__(P::T) void plane2_fwd_kernel(const typename Elem<DT
   }
 }
 
-// gk: the filter gradient, or with part != 0 the workgroup's share of it at part[(z H + h) K0 K2] (z = blockIdx.y),
-// summed by plane2_reduce_kernel.  GATED: x is q, gy the gradient of the gated output, gx receives dq.
+// gk: the filter gradient, or with part != 0 the workgroup's share of it at part[blockIdx.x K0 K2] (blockIdx.x =
+// share H + h), summed by plane2_reduce_kernel.  GATED: x is q, gy the gradient of the gated output, gx receives dq.
 template <int DT, class P, bool GATED>
 __global__ __launch_bounds__(P::T) void plane2_bwd_kernel(const typename Elem<DT>::T* __restrict__ gy,
                                                           const typename Elem<DT>::T* __restrict__ x,
@@ -418,7 +419,8 @@ __global__ __launch_bounds__(P::T) void plane2_bwd_kernel(const typename Elem<DT
   float2* lds = reinterpret_cast<float2*>(plane2_sm);
   const Plane2Io<DT, P, GATED> io(g, plane2_sm);
   const Plane2Roots<P> tw(lds + P::F0 * P::RS, roots);
-  const int h = int(blockIdx.x), b0 = int(blockIdx.y) * g.per_wg, b1 = min(g.B, b0 + g.per_wg);
+  const int share = int(blockIdx.x / unsigned(g.H)), h = int(blockIdx.x) - share * g.H;
+  const int b0 = share * g.per_wg, b1 = min(g.B, b0 + g.per_wg);
   const int64_t hk = g.kfilm ? int64_t(b0) * g.H + h : h;
   Plane2Vec<DT> xv[4], gv[4], kg[4], vv[4];
   const auto load = [&](int b) {
@@ -512,7 +514,7 @@ __global__ __launch_bounds__(P::T) void plane2_bwd_kernel(const typename Elem<DT
     __syncthreads();
   }
   const int64_t size = int64_t(g.K0) * g.K2;
-  const Plane2Filter kr(part ? part + (int64_t(blockIdx.y) * g.H + h) * size : gk + hk * size, g.K0, g.K2);
+  const Plane2Filter kr(part ? part + int64_t(blockIdx.x) * size : gk + hk * size, g.K0, g.K2);
   const auto put = [&](int row, int p, float c) {
     c *= scale;
     const int n2 = plane2_lag<P>(p, g.o2, c);

@@ -20,7 +20,8 @@ int nd_fwd(int nd, const void* x, const float* k, const void* shortcut, void* y,
   float2* ws = (float2*)workspace;
   const bool save = workspace_bytes >= nd_workspace_bytes(nd, B, H, S, K, kbatch, periodic, NSQ_DIR_BWD);
   Plane2Size z;
-  if (plane2_size(p, z)) {  // keeps no state: its backward transforms x and k again, in LDS
+  // keeps no state: its backward transforms x and k again, in LDS
+  if (plane2_size(p, z) && (plane2_bwd_ok(p, z) || !save)) {
     plane2_fwd(dtype, p, z, x, k, shortcut, y, nullptr, tw, st);
     NSQ_CHECK_LAUNCH();
     return NSQ_OK;
@@ -53,7 +54,7 @@ int nd_bwd(int nd, const void* g, const void* x, const float* k, const void* sho
   hipStream_t st = (hipStream_t)stream;
   float2* ws = (float2*)workspace;
   Plane2Size z;
-  if (plane2_size(p, z)) {
+  if (plane2_size(p, z) && plane2_bwd_ok(p, z)) {
     plane2_bwd(dtype, p, z, g, x, k, shortcut, gx, gk, gs, ws, nullptr, tw, st);
     NSQ_CHECK_LAUNCH();
     return NSQ_OK;

@@ -27,11 +27,12 @@ static int64_t nd_numel(int nd, int64_t B, int64_t H, const int64_t* S) {
 // results: the fused loaders and epilogues round as gate_ew_kernel does).
 // Small planes (plane2_size) form the gates as images enter and leave their kernels, but for the largest in fp32, whose
 // 1024-thread adjoint has no registers for the gates' operands (B=8 H=256 85 x 85: 673 us, 606 with the passes).
-static bool gated_fused_ok(const NdPlan& p, int dtype) {
+static bool gated_fused_ok(const NdPlan& p, int dtype, int direction) {
   const char* e = getenv("NSQ_ND_GATES_FUSED");
   if (e && e[0] == '0') return false;
   Plane2Size z;
-  if (plane2_size(p, z)) return !(dtype == NSQ_DTYPE_F32 && z.lF0 + z.lM == 13);
+  if (plane2_size(p, z) && (direction == NSQ_DIR_FWD || plane2_bwd_ok(p, z)))
+    return !(dtype == NSQ_DTYPE_F32 && z.lF0 + z.lM == 13);
   if (p.nd == 3) return plane_ok(p);
   return p.pack && p.o[2] % 2 == 0 && p.S[2] % 8 == 0;
 }
@@ -41,7 +42,7 @@ static size_t gated_nd_workspace_bytes(int nd, int64_t B, int64_t H, const int64
   const size_t conv = nd_workspace_bytes(nd, B, H, S, K, kbatch, periodic, direction);
   if (!conv || !valid_dtype(dtype)) return 0;
   NdPlan p;
-  if (make_nd_plan(nd, B, H, S, K, kbatch, periodic, p) && gated_fused_ok(p, dtype)) return conv;
+  if (make_nd_plan(nd, B, H, S, K, kbatch, periodic, p) && gated_fused_ok(p, dtype, direction)) return conv;
   const size_t es = dtype == NSQ_DTYPE_F32 ? 4 : 2;
   return round256(conv) + size_t(direction == NSQ_DIR_BWD ? 3 : 2) * round256(size_t(nd_numel(nd, B, H, S)) * es);
 }
@@ -86,7 +87,7 @@ static int gated_nd_fwd(int nd, const void* q, const void* kgate, const void* v,
   NSQ_CHECK_ARG(workspace && workspace_bytes >= need, "gated_fftconv_nd_fwd: workspace of %zu bytes required, got %zu",
                 need, workspace_bytes);
   hipStream_t st = (hipStream_t)stream;
-  if (gated_fused_ok(p, dtype)) {
+  if (gated_fused_ok(p, dtype, NSQ_DIR_FWD)) {
     const float2* tw = twiddle_table();
     if (!tw) return NSQ_ERR_HIP;
     const GatedIO gi{q, kgate, v, nullptr, y1, nullptr, nullptr, act1, act2};
@@ -138,12 +139,12 @@ static int gated_nd_bwd(int nd, const void* g, const void* q, const void* kgate,
   NSQ_CHECK_ARG(workspace && workspace_bytes >= need, "gated_fftconv_nd_bwd: workspace of %zu bytes required, got %zu",
                 need, workspace_bytes);
   hipStream_t st = (hipStream_t)stream;
-  if (gated_fused_ok(p, dtype)) {
+  if (gated_fused_ok(p, dtype, NSQ_DIR_BWD)) {
     const float2* tw = twiddle_table();
     if (!tw) return NSQ_ERR_HIP;
     const GatedIO gi{q, kgate, v, y1, nullptr, dv, dkgate, act1, act2};
     Plane2Size z;
-    if (plane2_size(p, z)) {
+    if (plane2_size(p, z) && plane2_bwd_ok(p, z)) {
       plane2_bwd(dtype, p, z, g, q, k, shortcut, dq, gk, gs, workspace, &gi, tw, st);
       NSQ_CHECK_LAUNCH();
       return NSQ_OK;

@@ -677,14 +677,59 @@ inline int validate_nd(int nd, const void* a, const void* b, const float* k, int
   return NSQ_OK;
 }
 
+// Small planes with whole images in LDS (fftconv2d_plane_*.hip): transform lengths 2^lF0 and 2^(lM + 1).
+struct Plane2Size {
+  int lF0, lM;
+};
+// The plane of a plan's shape, if this path takes it: zero-padded last axis, axis 0 zero-padded or periodic of at
+// least 16 points, transform lengths (the powers of two that hold the linear extent) of at most 128.  Where the
+// mixed-radix plan takes 96 x 96 the 128 x 128 plane (1024 threads, spills in the adjoint) is no faster (B=16 H=256
+// 48 x 48: 381 / 367 us forward + backward).  The other planes are in the forward, 1.1 to 3 times over 1500 shapes of 8
+// to 110 a side (24 x 24, 64 x 64 against 48 x 48: 60 / 95).
+inline bool plane2_size(const NdPlan& p, Plane2Size& z) {
+  if (p.nd != 2 || p.r[2] != 0 || p.wm[0] != -1 || p.wm[2] != -1) return false;
+  if (p.o[2] == 0 && p.F[2] == p.S[2]) return false;  // periodic, one tap
+  const bool per0 = p.o[0] == 0 && p.F[0] == p.S[0];
+  z.lF0 = per0 ? p.lF[0] : ilog2_ceil(int64_t(p.S[0]) + (p.K[0] + 1) / 2);
+  z.lM = ilog2_ceil(int64_t(p.S[2]) + (p.K[2] + 1) / 2) - 1;
+  if (z.lF0 < 4) z.lF0 = 4;
+  if (z.lM < 3) z.lM = 3;
+  if (z.lF0 + z.lM < 9) {  // at least one wave of 8 points a lane
+    if (per0)
+      z.lM = 9 - z.lF0;
+    else
+      z.lF0 = 9 - z.lM;
+  }
+  if (p.kb != 1 && p.B * p.H >= (int64_t(1) << (34 - z.lF0 - z.lM))) return false;  // threads of a launch: 2^32
+  return z.lF0 <= 7 && z.lM <= 6 && !(p.r3 && z.lF0 + z.lM == 13);
+}
+// The adjoint, if the forward has a plane: not where the mixed-radix plan takes 96 x 48 or 48 x 96, 1.78 times fewer
+// points than 128 x 64, and the images fill the GPU (backward, us, passes / plane: B=32 H=256 53 x 34 gated 372 / 500,
+// B=64 H=64 17 x 45 115 / 144; at B H = 2048 the plane is 1.05 to 1.26 times faster, below more).  A training forward
+// then runs the passes too, whose state that backward takes.
+inline bool plane2_bwd_ok(const NdPlan& p, const Plane2Size& z) {
+  return !(p.r3 && z.lF0 + z.lM == 12 && p.B * p.H >= 3072);
+}
+// Shares of a channel's batch at most: 2^25 points in all workgroups, four rounds of the GPU or more.
+inline int64_t plane2_max_split(const NdPlan& p, const Plane2Size& z) {
+  const int64_t n = (int64_t(1) << (24 - z.lF0 - z.lM)) / p.H;
+  return p.kb != 1 || n < 1 ? 1 : n < p.B ? n : p.B;
+}
+
+// direction NSQ_DIR_STATE: what a forward may leave for the backward (a backward-sized workspace), 0 if nothing.
 inline size_t nd_workspace_bytes(int nd, int64_t B, int64_t H, const int64_t* S, const int64_t* K, int64_t kbatch,
                                  unsigned periodic, int direction) {
   NdPlan p;
   if (!S || !K || !make_nd_plan(nd, B, H, S, K, kbatch, periodic, p)) return 0;
-  const int64_t blocks = direction == NSQ_DIR_BWD
-                             ? (2 * B * H + (1 + bwd_batch_split(p)) * kbatch * H)
-                             : (B * H + kbatch * H);
-  return size_t(blocks * p.spec) * sizeof(float2);
+  const size_t fwd = size_t((B * H + kbatch * H) * p.spec) * sizeof(float2);
+  if (direction == NSQ_DIR_FWD) return fwd;
+  Plane2Size z;
+  if (plane2_size(p, z) && plane2_bwd_ok(p, z)) {  // the shares' filter gradients; a forward takes this workspace too
+    if (direction == NSQ_DIR_STATE) return 0;
+    const size_t shares = size_t(plane2_max_split(p, z) * H) * p.K[0] * p.K[2] * sizeof(float);
+    return shares > fwd ? shares : fwd;
+  }
+  return size_t((2 * B * H + (1 + bwd_batch_split(p)) * kbatch * H) * p.spec) * sizeof(float2);
 }
 
 // The run_nd_* instances are compiled once each, in fftconv_nd_{f32,bf16,f16}.hip
@@ -703,30 +748,6 @@ NSQ_ND_RUN_INSTANCES(extern, NSQ_DTYPE_F32, true)
 NSQ_ND_RUN_INSTANCES(extern, NSQ_DTYPE_BF16, true)
 NSQ_ND_RUN_INSTANCES(extern, NSQ_DTYPE_F16, true)
 
-// Small planes with whole images in LDS (fftconv2d_plane_*.hip): transform lengths 2^lF0 and 2^(lM + 1).
-struct Plane2Size {
-  int lF0, lM;
-};
-// The plane of a plan's shape, if this path takes it: zero-padded last axis, axis 0 zero-padded or periodic of at
-// least 16 points, transform lengths (the powers of two that hold the linear extent) of at most 128.  Where the
-// mixed-radix plan takes 96 x 96 the 128 x 128 plane (1024 threads, spills in the adjoint) is no faster (B=16 H=256
-// 48 x 48: 381 / 367 us forward + backward); every smaller plane is (24 x 24, 64 x 64 against 48 x 48: 60 / 95).
-inline bool plane2_size(const NdPlan& p, Plane2Size& z) {
-  if (p.nd != 2 || p.r[2] != 0 || p.wm[0] != -1 || p.wm[2] != -1) return false;
-  if (p.o[2] == 0 && p.F[2] == p.S[2]) return false;  // periodic, one tap
-  const bool per0 = p.o[0] == 0 && p.F[0] == p.S[0];
-  z.lF0 = per0 ? p.lF[0] : ilog2_ceil(int64_t(p.S[0]) + (p.K[0] + 1) / 2);
-  z.lM = ilog2_ceil(int64_t(p.S[2]) + (p.K[2] + 1) / 2) - 1;
-  if (z.lF0 < 4) z.lF0 = 4;
-  if (z.lM < 3) z.lM = 3;
-  if (z.lF0 + z.lM < 9) {  // at least one wave of 8 points a lane
-    if (per0)
-      z.lM = 9 - z.lF0;
-    else
-      z.lF0 = 9 - z.lM;
-  }
-  return z.lF0 <= 7 && z.lM <= 6 && !(p.r3 && z.lF0 + z.lM == 13);
-}
 // gate: the Hyena gates' operands (x is then q; gated_nd_fwd / gated_nd_bwd), or null.
 template <int DT>
 void plane2_fwd(const NdPlan& p, const Plane2Size& z, const void* x, const float* k, const void* s, void* y,

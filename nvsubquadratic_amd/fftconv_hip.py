@@ -473,13 +473,14 @@ def fftconv_nd_bwd_raw(g, x, k, s, gx, gk, gs, kbatch: int, workspace: torch.Ten
 
 
 def _nd_state_bytes(x: torch.Tensor, k: torch.Tensor, kbatch: int, periodic: int, keep: bool) -> int:
+    """Bytes of forward state a training forward keeps: 0 too where the shape's forward leaves none."""
     if not keep:
         return 0
     nd = x.ndim - 2
     return _within_budget(
         int(_nd_workspace_bytes(_lib.get_lib(), nd, int(x.shape[0]), int(x.shape[1]),
                                 _lib.i64_array([int(d) for d in x.shape[2:]]),
-                                _lib.i64_array([int(d) for d in k.shape[1:]]), kbatch, periodic, _lib.NSQ_DIR_BWD)),
+                                _lib.i64_array([int(d) for d in k.shape[1:]]), kbatch, periodic, _lib.NSQ_DIR_STATE)),
         x.device)
 
 

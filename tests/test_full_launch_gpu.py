@@ -17,10 +17,12 @@ the heuristic cannot silently move a test off the path it is meant for):
 * config 4 (B=16, C=384, 128^2, filter 128^2, F = 256^2): product pass 8
   images per workgroup, adjoint 16;
 * config 5 (B=2, C=128, 64^3, F = 128^3): 2 images per workgroup both ways;
-* 2D B=2, H=2048, 32^2, filter 32^2 (F = 64^2): bsplit = 1, 2 images per
-  workgroup both ways;
-* 2D B=8, H=512, 64^2, filter 64^2 (F = 128^2): product bsplit = 3, runs of
-  3, 3 and 2 images; adjoint 8 images.
+* 2D B=7, H=2048, 140 x 20, filter 140 x 20 (F = 256 x 32): product bsplit
+  = 3, runs of 3, 3 and 1 images; adjoint 7 images;
+* 2D B=2, H=2048, 32^2, filter 32^2 and B=8, H=512, 64^2, filter 64^2: the
+  split of these passes is mirrored too, but planes of up to 128 x 128 and the
+  mixed-radix lengths run other kernels (test_fftconv2d_plane_gpu.py has those
+  with several images a workgroup).
 
 Tolerances: rel-L2 <= 1e-4 fp32, <= 2e-2 bf16 I/O against the float32 oracle,
 plus a 5e-3 check of bf16 outputs against the float64 restatement.
@@ -91,6 +93,7 @@ def _check_nd_full(x, k, s, g, fn, tol, tol64=None):
 @pytest.mark.parametrize("B,H,S,K,fwd_imgs,bwd_imgs", [
     (2, 2048, (32, 32), (32, 32), 2, 2),  # bsplit = 1 both ways
     (8, 512, (64, 64), (64, 64), 3, 8),   # product pass runs of 3, 3, 2 images
+    (7, 2048, (140, 20), (140, 20), 3, 7),  # on these passes: runs of 3, 3, 1 images
 ])
 def test_2d_multi_image_axis0_workgroups_fp32(B, H, S, K, fwd_imgs, bwd_imgs):
     assert _images_per_workgroup(B, H, S, K, adjoint=False) == fwd_imgs
