@@ -49,20 +49,20 @@ struct RingCfg {
   static_assert(LOGM >= 9 && LOGM <= 13, "RingCfg: length out of range");
 };
 
-// W_32^r, r < 8 (correctly rounded).
-__device__ constexpr float kRingCos[9] = {1.f,
-                                          0.98078528040323044913f,
-                                          0.92387953251128675613f,
-                                          0.83146961230254523708f,
-                                          0.70710678118654752440f,
-                                          0.55557023301960222474f,
-                                          0.38268343236508977173f,
-                                          0.19509032201612826785f,
-                                          0.f};
-template <int LOGR>
-__device__ __forceinline__ float2 ring_rot(int r) {  // W_{4R}^r
-  const int i = r << (3 - LOGR);
-  return make_float2(kRingCos[i], -kRingCos[8 - i]);
+// W_{4M}^n, n < M, correctly rounded (M = 8192: beyond the table's 2^14 segment, odd n are one product more).  Every
+// sample meets one on its way in and out: as products of two rounded roots they cost a tenth of the transform's error
+// (2.50e-7 against 2.19e-7 of the packed transform at B=2 H=128 L=4096 fp32).
+template <class C>
+__device__ __forceinline__ float2 ring_fold(const float2* __restrict__ tw, int n) {
+  constexpr int LOGB = C::LOGM + 2;
+  if constexpr (LOGB <= 14) {
+    return tw[(1 << LOGB) + n];
+  } else {
+    static_assert(LOGB == 15, "ring_fold: roots of unity");
+    const float2 e = tw[(1 << 14) + (n >> 1)];
+    const float2 o = cmul_fixed(e, make_float2(1.f, -1.91747597e-4f));  // W_32768
+    return n & 1 ? o : e;
+  }
 }
 
 // One pass over the thread's 8 points: ld(i, j, v) reads butterfly j's inputs, st(i, base, v) takes outputs base + r NS.
@@ -125,16 +125,16 @@ struct RingRow {
 };
 
 // A row -> the thread's 8 spectral points: lo(i, r, n) is the sample n = tid + i T + r M / R, hi(n) samples from M on
-// (WIDE).
-template <class C, bool WIDE, class LO, class HI>
+// (WIDE).  TABLE: the last pass's roots all from the table, not four of seven as products (fp32 rows: their results show
+// it, 16-bit ones do not).
+template <class C, bool WIDE, bool TABLE = false, class LO, class HI>
 __device__ __forceinline__ void ring_spectrum(float2* lds, LO&& lo, HI&& hi, float2 (&v)[8],
                                               const float2* __restrict__ tw) {
   ring_pass<C::LOGM, C::R0, 0, false, C::T>(
       [&](int i, int j, float2 (&z)[C::R]) {
-        const float2 w0 = root<C::LOGM + 2>(tw, j);
 #pragma unroll
         for (int r = 0; r < C::R; ++r) {
-          const float2 w = cmul_fixed(w0, ring_rot<C::R0>(r));
+          const float2 w = ring_fold<C>(tw, j + r * C::NR);
           const float a = lo(i, r, j + r * C::NR), c = WIDE ? hi(j + r * C::NR + C::M) : 0.f;
           z[r] = make_float2(fmaf(c, w.y, a * w.x), fmaf(-c, w.x, a * w.y));
         }
@@ -147,7 +147,12 @@ __device__ __forceinline__ void ring_spectrum(float2* lds, LO&& lo, HI&& hi, flo
   ring_middle<C, C::R0, false>(lds, tw);
   const int j = opaque_tid();
   float2 w[8];
-  pass_twiddles<8>(TwTable(tw), C::M, j, w);
+  if constexpr (TABLE) {
+#pragma unroll
+    for (int r = 1; r < 8; ++r) w[r] = TwTable(tw).load(C::M, (r * j) & (C::M - 1));
+  } else {
+    pass_twiddles<8>(TwTable(tw), C::M, j, w);
+  }
   const float2* q = lds + pad16(j);
   v[0] = q[0];
 #pragma unroll
@@ -174,10 +179,9 @@ __device__ __forceinline__ void ring_inverse(float2* lds, float2 (&v)[8], OUT&& 
         for (int r = 0; r < C::R; ++r) z[r] = q[pad16(r * C::NR)];
       },
       [&](int, int base, const float2 (&z)[C::R]) {  // base = j < NR: outputs j + r NR
-        const float2 w0 = root<C::LOGM + 2>(tw, base);
 #pragma unroll
         for (int r = 0; r < C::R; ++r) {
-          const float2 a = cmulc(z[r], cmul_fixed(w0, ring_rot<C::R0>(r)));
+          const float2 a = cmulc(z[r], ring_fold<C>(tw, base + r * C::NR));
           out(base + r * C::NR, a.x, -a.y);
         }
       },
@@ -211,7 +215,7 @@ __global__ __launch_bounds__(RingCfg<LOGM>::T) __attribute__((amdgpu_waves_per_e
     const RowBuf<NSQ_DTYPE_F32, false> kb(k + hk * K, K);
     RingRow<NSQ_DTYPE_F32, C> kr;
     kr.load(kb);
-    ring_spectrum<C, WIDE>(
+    ring_spectrum<C, WIDE, DT == NSQ_DTYPE_F32>(
         lds, [&](int i, int r, int) { return __uint_as_float(kr.w[i][r]); }, [&](int n) { return kb.elem(n); }, kv,
         tw);
   }
@@ -223,7 +227,7 @@ __global__ __launch_bounds__(RingCfg<LOGM>::T) __attribute__((amdgpu_waves_per_e
     const RowBuf<DT, false> xb = row(x, b), kb = row(GATE ? ga.kg : x, b), yb = row(y, b);
     const auto z = [&](int n) { return GATE ? gate1<DT>(ga.act1, xb.elem(n), kb.elem(n)) : xb.elem(n); };
     float2 v[8];
-    ring_spectrum<C, WIDE>(
+    ring_spectrum<C, WIDE, DT == NSQ_DTYPE_F32>(
         lds,
         [&](int i, int r, int) {
           const float a = RowBuf<DT, false>::bits_to_f32(rx.w[i][r]);

@@ -18,6 +18,7 @@ import pytest
 import torch
 
 from nvsubquadratic_amd import fftconv_hip as F
+from nvsubquadratic_amd.gated_fftconv_hip import hyena_gated_causal_fftconv1d_bhl
 from nvsubquadratic_amd.workloads import causal1d_case
 from oracle.fftconv_ref import causal_fftconv1d_np, causal_fftconv1d_torch, rel_l2
 
@@ -261,36 +262,43 @@ def test_config1_fp32_fwd_bwd():
     assert rel_l2(s.grad, sg.grad) < RTOL_F32_L2
 
 
-@pytest.mark.parametrize("L", [2048, 4096, 8192])
-@pytest.mark.parametrize("dtype,film", [(torch.float32, False), (torch.bfloat16, False), (torch.float32, True)])
-def test_fused_pair_and_single_kernels_agree(L, dtype, film):
-    """The fused forward runs up to 1536 / 1536 / 256 rows (B*H) of FFT lengths 4096 / 8192 / 16384 on the
-    two-transform (filter | row) workgroup and larger grids on the one-transform kernel: 8 channels past that bound
-    take the latter, the bound's worth of them the former.  At FFT length 16384 both run radix-16 passes and agree
-    bit for bit; up to 8192 the pair kernel runs radix-8 passes (8 points per thread, twice the threads), so the two
-    agree to fp32 rounding (rel-L2 <= 1e-6 on fp32 outputs; <= 1e-3 on bf16 outputs, where a rounding difference can
-    move an output by one bf16 step) and the pair kernel repeats bit for bit.  Both meet the oracle."""
-    torch.manual_seed(31)
-    B = 2 if film else 1
-    rows = {2048: 1536, 4096: 1536, 8192: 256}[L]
-    H, Hp = rows // B + 8, rows // B
-    x = torch.randn(B, H, L).to(dtype)
-    k = torch.randn(B if film else 1, H, L) * torch.exp(-torch.linspace(0, 8, L))
-    s = torch.randn(H).to(dtype)
-    xd, kd, sd = x.cuda(), k.cuda(), s.cuda()
-    y_single = F.causal_fftconv1d_bhl(xd, kd, sd)
-    y_pair = F.causal_fftconv1d_bhl(xd[:, :Hp].contiguous(), kd[:, :Hp].contiguous(), sd[:Hp].contiguous())
-    if L == 8192:
-        assert torch.equal(y_pair, y_single[:, :Hp])
-    else:
-        assert rel_l2(y_single[:, :Hp], y_pair) < (1e-6 if dtype == torch.float32 else 1e-3)
-        y_again = F.causal_fftconv1d_bhl(xd[:, :Hp].contiguous(), kd[:, :Hp].contiguous(), sd[:Hp].contiguous())
-        assert torch.equal(y_pair, y_again)
+@pytest.mark.parametrize("B,H,L,film", [(5, 1000, 2048, False), (5, 600, 8192, False), (5, 1100, 700, False),
+                                        (2, 768, 2048, True), (3, 40, 4096, False)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_ring_rows_of_a_workgroup_agree_with_single_rows(B, H, L, film, dtype):
+    """A workgroup of the ring forward takes one row of its channel after the other once the grid has 2^19 threads
+    (F / 16 each): two of five with a single last one, or all five.  Each row is what a call with that row alone gives,
+    bit for bit; sampled channels against float64.  Where few enough elements are gated in the kernel, the same with the
+    gates.  Per-sample filters and small grids: one row a workgroup."""
+    fft = 1 << (2 * L - 1 - 1).bit_length()
+    shares = 1 if film else min(B, -(-(1 << 19) // (fft // 16) // H))
+    assert film or (-(-B // shares) > 1) == (H >= 600)
+    gen = torch.Generator(device="cuda").manual_seed(H)
+    x, kg, v = (torch.randn(B, H, L, device="cuda", generator=gen).to(dtype) for _ in range(3))
+    k = torch.randn(B if film else 1, H, L, device="cuda", generator=gen)
+    k *= torch.exp(-torch.linspace(0, 8, L, device="cuda"))
+    s = torch.randn(H, device="cuda", generator=gen).to(dtype)
     tol = RTOL_F32_L2 if dtype == torch.float32 else RTOL_BF16_L2
-    y64 = np.concatenate([causal_fftconv1d_np(x[b:b + 1].float().numpy(), k[b if film else 0].numpy(),
-                                              s.float().numpy()) for b in range(B)])
-    assert rel_l2(y64, y_single) < tol
-    assert rel_l2(y64[:, :Hp], y_pair) < tol
+    ch = torch.tensor([0, H // 2 + 1, H - 1], device="cuda")
+
+    def conv64(z):
+        kf = torch.fft.rfft(k[:, ch].double(), n=2 * L)
+        return torch.fft.irfft(torch.fft.rfft(z, n=2 * L) * kf, n=2 * L)[..., :L] + s[ch].double().view(1, -1, 1) * z
+
+    y = F.causal_fftconv1d_bhl(x, k, s)
+    for b in range(B):
+        one = F.causal_fftconv1d_bhl(x[b:b + 1].contiguous(), k[b:b + 1].contiguous() if film else k, s)
+        assert torch.equal(y[b:b + 1], one), b
+    assert rel_l2(conv64(x[:, ch].double()).cpu(), y[:, ch].cpu()) < tol
+    if B * H * L >= 1 << 22 or film:
+        return
+    y = hyena_gated_causal_fftconv1d_bhl(x, kg, v, k, s, "silu")
+    for b in range(B):
+        one = hyena_gated_causal_fftconv1d_bhl(*(t[b:b + 1].contiguous() for t in (x, kg, v)), k, s, "silu")
+        assert torch.equal(y[b:b + 1], one), b
+    q6, k6, v6 = (t[:, ch].double() for t in (x, kg, v))
+    silu = torch.nn.functional.silu
+    assert rel_l2((conv64(q6 * silu(k6)) * silu(v6)).cpu(), y[:, ch].cpu()) < 2 * tol
 
 
 def test_config3_channel_sample_bf16_fwd_bwd():
