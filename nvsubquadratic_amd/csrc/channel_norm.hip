@@ -520,6 +520,14 @@ template <int DT>
 bool norm16_ok(int C, int64_t S, std::initializer_list<const void*> ptrs) {
   return DT != NSQ_DTYPE_F32 && C <= kNorm16MaxC && C * S < (int64_t(1) << 30) && use_vec(8, C, S, 8, ptrs);
 }
+// Where they are the faster ones, tile kernel / register kernel in us: not forward at 65 to 80 channels, which leave 40%
+// of the 128 a workgroup holds empty (C = 72, 16 x 16384 positions 36.0 / 40.8; C = 96 is faster); with few positions
+// not above 768 channels (C = 1000, 256 positions, forward + backward 36.8 / 38.9) and, whose vectors spill, above 1024
+// (C = 1280, 1024 positions forward 12.2 / 14.4; C = 1536 backward, 784 positions 70 / 77, 25088 748 / 249).
+inline bool norm16_pays(bool bwd, int C, int64_t positions) {
+  if (C > 768 && positions < (C > 1024 ? 4096 : 512)) return false;
+  return bwd || C <= 64 || C > 80;
+}
 template <int DT, bool BWD, class F>
 void with_norm16_kernel(int C, bool gated, int act, int mode, F&& f) {
   if constexpr (DT != NSQ_DTYPE_F32)
@@ -551,7 +559,7 @@ template <int DT>
 void launch_fwd(const void* y, const void* v, const float* w, void* out, int64_t B, int C, int64_t S, float eps,
                 int gated, int act, int out_blh, hipStream_t st, int mode = CHN_RMS, const float* bias = nullptr) {
   constexpr int VW = 16 / int(sizeof(typename Elem<DT>::T));
-  if (norm16_ok<DT>(C, S, {y, v, out})) {
+  if (norm16_ok<DT>(C, S, {y, v, out}) && norm16_pays(false, C, B * S)) {
     with_norm16_kernel<DT, false>(C, gated, act, mode, [&](auto cfg, auto mc, auto gt) {
       using T = typename Elem<DT>::T;
       using F = decltype(cfg);
@@ -592,9 +600,7 @@ void launch_bwd(const void* dout, const void* y, const void* v, const float* w, 
   constexpr int VW = 16 / int(sizeof(typename Elem<DT>::T));
   float* partb = (mode == CHN_LN && db) ? part + p.nwg * int64_t(C) : nullptr;
   int64_t nwg = p.nwg;
-  // above 1024 channels a lane's vectors spill: a few tiles run no faster than the tile kernel (C = 1536, 784
-  // positions: 77 / 70 us; 25088: 249 / 748)
-  if (norm16_ok<DT>(C, S, {dout, y, v, dy, dv}) && (C <= 1024 || B * S >= 4096)) {
+  if (norm16_ok<DT>(C, S, {dout, y, v, dy, dv}) && norm16_pays(true, C, B * S)) {
     with_norm16_kernel<DT, true>(C, gated, act, mode, [&](auto cfg, auto mc, auto gt) {
       using T = typename Elem<DT>::T;
       using F = decltype(cfg);
