@@ -785,8 +785,9 @@ static float* noalloc_scratch() {
 }
 
 // What the noalloc entry point counts against its scratch, which fixes the shapes it takes: partials of one run per
-// kConvSegTiles tiles, and for silu above 16 taps an fp32 row set [B, C, L].  Never less than the backward
-// uses where that fits (at most max(C, 4096 + C) partial rows).
+// kConvSegTiles tiles, and for silu above 16 taps an fp32 row set [B, C, L] that no kernel needs any more (the entry
+// point's shapes stay what they were).  Never less than the backward uses where that fits (at most max(C, 4096 + C)
+// partial rows).
 static size_t noalloc_bytes(int64_t B, int64_t C, int64_t L, int64_t K, int act) {
   const int64_t pre = act == NSQ_ACT_SILU && K > 16 ? B * C * L : 0;
   const size_t was = size_t(pre + C * cconv_wgrad_parts(B, L) * (K + 1)) * sizeof(float);
@@ -848,9 +849,8 @@ int nsq_causal_conv1d_bwd(const void* gy, const void* x, const float* weight, co
   return NSQ_OK;
 }
 
-// The scratch regions the backward uses (partials, the silu pre-activation
-// gradient) are written in full by one kernel before the next reads them, so
-// the buffer needs no clearing between calls.
+// The partials are written in full by one kernel before the next reads them,
+// so the buffer needs no clearing between calls.
 int nsq_causal_conv1d_bwd_noalloc(const void* gy, const void* x, const float* weight, const float* bias, void* gx,
                                   float* gweight, float* gbias, int dtype, int activation, int64_t B, int64_t C,
                                   int64_t L, int64_t K, void* stream) {

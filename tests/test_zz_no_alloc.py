@@ -4,9 +4,9 @@ workspace entry point it mirrors (nsq_causal_conv1d_bwd), both called through th
 Both run the same kernels in the same order, so the outputs must agree bitwise.  Two calls
 in a row on the shared device scratch, the second with a smaller input, show that nothing
 from the first call leaks into the second; shapes cover the register path (K <= 16, only
-weight / bias partials in scratch) and the matrix-core path with silu (K > 16, where the
-pre-activation gradient lives in scratch too).  A shape whose scratch exceeds the fixed
-buffer is refused on the host with NSQ_ERR_UNSUPPORTED.
+weight / bias partials in scratch) and the matrix-core path with silu (K > 16, which also keeps
+partials only).  A shape whose scratch exceeds the fixed buffer is refused on the host with
+NSQ_ERR_UNSUPPORTED.
 """
 
 import pytest
