@@ -159,18 +159,17 @@ __device__ __forceinline__ void load_tile_u(const typename Elem<DT>::T* __restri
 #pragma unroll
   for (int k = 0; k < VW; ++k) red[m.g * TS + p0 + k] = ss[k];
   __syncthreads();
-  const bool inside = s0 + int(threadIdx.x) < S;
   if (threadIdx.x < TS) {
     float sum = 0.f;
     for (int k = 0; k < m.G; ++k) sum += red[k * TS + threadIdx.x];
     if (mode == CHN_L2) {
       const float n = Elem<DT>::round(sqrtf(sum));
-      rs[threadIdx.x] = inside ? 1.f / fmaxf(n, eps) : 0.f;
+      rs[threadIdx.x] = s0 + int(threadIdx.x) < S ? 1.f / fmaxf(n, eps) : 0.f;
       if (cl) cl[threadIdx.x] = n < eps ? 0.f : 1.f;
     } else if (mode == CHN_LN) {
       rs[threadIdx.x] = sum / float(C);  // the mean, until the second sweep
     } else {
-      rs[threadIdx.x] = inside ? rsqrtf(sum * (1.f / float(C)) + eps) : 0.f;
+      rs[threadIdx.x] = s0 + int(threadIdx.x) < S ? rsqrtf(sum * (1.f / float(C)) + eps) : 0.f;
     }
   }
   __syncthreads();
@@ -192,7 +191,7 @@ __device__ __forceinline__ void load_tile_u(const typename Elem<DT>::T* __restri
     if (threadIdx.x < TS) {
       float sum = 0.f;
       for (int k = 0; k < m.G; ++k) sum += red[k * TS + threadIdx.x];
-      rs[threadIdx.x] = inside ? rsqrtf(sum * (1.f / float(C)) + eps) : 0.f;
+      rs[threadIdx.x] = s0 + int(threadIdx.x) < S ? rsqrtf(sum * (1.f / float(C)) + eps) : 0.f;
     }
     __syncthreads();
   }
