@@ -30,10 +30,12 @@
 //   4 x 1024 x 8192      239 -> 166      513 -> 314
 //   1 x  256 x 8192     24.3 ->  20.3     45 ->  30
 //   1 x   64 x 4096     13.4 ->  10.8
+// with the fold's roots as products (ring_fold); from the table, as now, 2 % more at L = 8192 and 512, 8 to 13 % between.
 // fp32 within 6 % of these.  Small grids ran two transforms side by side in
-// one workgroup before (the 1-row figures): the ring is faster there too, from
-// 64 rows to 1536, so it takes every grid size.  Error against float64 (B=2 H=128 L=4096 fp32): 2.5e-7, as fp32 FFTs
-// of this length give (2.2e-7 before).
+// one workgroup before (the 1-row figures): the ring is faster there too but for
+// 64 to 256 rows of F = 4096 with a short filter (9.3 -> 10.3), so it takes every
+// grid size.  Error against float64 (B=2 H=128 fp32), packed -> ring: y 1.84 -> 1.77e-7 at L = 512, 2.02 -> 2.05e-7 at
+// 2048, 2.16 -> 2.12e-7 at 4096, 2.49 -> 2.15e-7 at 8192; gx and gk below the packed transform's at every length.
 #pragma once
 
 #include "gate.h"
@@ -49,19 +51,22 @@ struct RingCfg {
   static_assert(LOGM >= 9 && LOGM <= 13, "RingCfg: length out of range");
 };
 
-// W_{4M}^n, n < M, correctly rounded (M = 8192: beyond the table's 2^14 segment, odd n are one product more).  Every
-// sample meets one on its way in and out: as products of two rounded roots they cost a tenth of the transform's error
-// (2.50e-7 against 2.19e-7 of the packed transform at B=2 H=128 L=4096 fp32).
+// W_{4M}^n of a first-pass butterfly's inputs n = j + r M / R, r < R.  Every sample meets one on its way in and out: as
+// products of two rounded roots they cost a tenth of the transform's error (2.46e-7 against 2.16e-7 of the packed
+// transform at B=2 H=128 L=4096 fp32), so they come from the table.  M = 8192 is beyond its 2^14 segment: there odd j
+// are one product (by W_32768), and r = 1 one more (W_8), still 2.3e-7 where the hardware's sine and cosine gave 3.2e-7
+// and the packed transform 2.5e-7 (L=8192); two table reads and a select a sample instead cost the backward 10%.
 template <class C>
-__device__ __forceinline__ float2 ring_fold(const float2* __restrict__ tw, int n) {
+__device__ __forceinline__ void ring_fold(const float2* __restrict__ tw, int j, float2 (&w)[C::R]) {
   constexpr int LOGB = C::LOGM + 2;
   if constexpr (LOGB <= 14) {
-    return tw[(1 << LOGB) + n];
+#pragma unroll
+    for (int r = 0; r < C::R; ++r) w[r] = tw[(1 << LOGB) + j + r * C::NR];
   } else {
-    static_assert(LOGB == 15, "ring_fold: roots of unity");
-    const float2 e = tw[(1 << 14) + (n >> 1)];
-    const float2 o = cmul_fixed(e, make_float2(1.f, -1.91747597e-4f));  // W_32768
-    return n & 1 ? o : e;
+    static_assert(LOGB == 15 && C::R == 2, "ring_fold: roots of unity");
+    const float2 e = tw[(1 << 14) + (j >> 1)];
+    w[0] = cmul_fixed(e, make_float2(1.f, j & 1 ? -1.91747597e-4f : 0.f));  // cos rounds to 1
+    w[1] = cmul_fixed(w[0], make_float2(0.70710678118654752440f, -0.70710678118654752440f));
   }
 }
 
@@ -132,9 +137,11 @@ __device__ __forceinline__ void ring_spectrum(float2* lds, LO&& lo, HI&& hi, flo
                                               const float2* __restrict__ tw) {
   ring_pass<C::LOGM, C::R0, 0, false, C::T>(
       [&](int i, int j, float2 (&z)[C::R]) {
+        float2 wf[C::R];
+        ring_fold<C>(tw, j, wf);
 #pragma unroll
         for (int r = 0; r < C::R; ++r) {
-          const float2 w = ring_fold<C>(tw, j + r * C::NR);
+          const float2 w = wf[r];
           const float a = lo(i, r, j + r * C::NR), c = WIDE ? hi(j + r * C::NR + C::M) : 0.f;
           z[r] = make_float2(fmaf(c, w.y, a * w.x), fmaf(-c, w.x, a * w.y));
         }
@@ -179,9 +186,11 @@ __device__ __forceinline__ void ring_inverse(float2* lds, float2 (&v)[8], OUT&& 
         for (int r = 0; r < C::R; ++r) z[r] = q[pad16(r * C::NR)];
       },
       [&](int, int base, const float2 (&z)[C::R]) {  // base = j < NR: outputs j + r NR
+        float2 wf[C::R];
+        ring_fold<C>(tw, base, wf);
 #pragma unroll
         for (int r = 0; r < C::R; ++r) {
-          const float2 a = cmulc(z[r], ring_fold<C>(tw, base + r * C::NR));
+          const float2 a = cmulc(z[r], wf[r]);
           out(base + r * C::NR, a.x, -a.y);
         }
       },
