@@ -30,11 +30,12 @@
 //   4 x 1024 x 8192      239 -> 166      513 -> 314
 //   1 x  256 x 8192     24.3 ->  20.3     45 ->  30
 //   1 x   64 x 4096     13.4 ->  10.8
-// with the fold's roots as products (ring_fold); from the table, as now, 2 % more at L = 8192 and 512, 8 to 13 % between.
+// with the fold's roots as products; from the table (ring_fold), as now, 2 % more
+// at L = 512 and 8192 and 8 to 13 % between.
 // fp32 within 6 % of these.  Small grids ran two transforms side by side in
 // one workgroup before (the 1-row figures): the ring is faster there too but for
 // 64 to 256 rows of F = 4096 with a short filter (9.3 -> 10.3), so it takes every
-// grid size.  Error against float64 (B=2 H=128 fp32), packed -> ring: y 1.84 -> 1.77e-7 at L = 512, 2.02 -> 2.05e-7 at
+// grid size.  Error against float64 (B=2 H=128 fp32), packed -> ring: y 1.86 -> 1.79e-7 at L = 512, 2.02 -> 2.05e-7 at
 // 2048, 2.16 -> 2.12e-7 at 4096, 2.49 -> 2.15e-7 at 8192; gx and gk below the packed transform's at every length.
 #pragma once
 
